@@ -17,22 +17,22 @@
 //             when causal).
 //   ctx     = probs.matmul(v), merged back to [B, T, H*hd].
 //
-// Three kernels, chosen per call:
-//  * flash_attn_tr_kernel (bf16/fp16, hd = 64, T % 8 == 0, power-of-two
-//    scale -- the scale is round(1/sqrt(64)) = 0.125 for every hd = 64 call):
-//    K and V tiles are copied to LDS in their natural layouts and the MFMA
-//    operands are read back transposed with ds_read_b64_tr_b16;
-//  * flash_attn_kernel (bf16/fp16, hd = 64, any T): transposes K and V while
-//    writing them to LDS, and applies both score roundings;
-//  * attn_generic_kernel (below).
-// Both flash kernels compute S^T = K*Q^T and O^T = V^T*P^T on
-// v_mfma_f32_16x16x32 so that every lane owns one query row: P goes from the
-// S accumulators into the PV operand without touching LDS.  Scores are
-// rounded like the reference (round(matmul), then round(*scale)).
+// Kernels, chosen per call (attention() below):
+//  * flash_attn_pipe_kernel (bf16/fp16, hd = 64, T % 64 == 0): the
+//    software-pipelined main path;
+//  * flash_attn_tr_kernel (bf16/fp16, hd <= 128, hd % 8 == 0, any T): K and V
+//    tiles are copied to LDS in their natural layouts and the MFMA operands
+//    are read back transposed with ds_read_b64_tr_b16;
+//  * attention_f32 (attention_f32.hip; fp32, hd <= 128, hd % 4 == 0);
+//  * attn_generic_kernel (below): every other head size or alignment.
+// The flash kernels compute S^T = K*Q^T and O^T = V^T*P^T so that every lane
+// owns one query row: P goes from the S accumulators into the PV operand
+// without touching LDS.  Scores are rounded like the reference
+// (round(matmul), then round(*scale)).
 //
-// Generic path (any dtype / head size): one wave per query row, scores kept in
-// LDS, float max / double sum / per-j float accumulation as the reference's
-// fp32 CPU kernels do (src/backend/cpu_backend.hpp:334-374, 587-611).
+// Generic path: one wave per query row, scores kept in LDS, float max /
+// double sum / per-j float accumulation as the reference's fp32 CPU kernels
+// do (src/backend/cpu_backend.hpp:334-374, 587-611).
 #include <cmath>
 #include <cstdlib>
 #include <string>
@@ -97,204 +97,14 @@ template <> __device__ __forceinline__ void round4<F16>(float v[4]) { round4_f16
 // c ^ (r & 7).
 __device__ __forceinline__ int swz(int r, int c) { return r * 8 + (c ^ (r & 7)); }
 
-template <int DT, int RW>
-__global__ void __launch_bounds__(256)
-flash_attn_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-                  uint16_t *__restrict__ O, int B, int H, int T, int causal, float scale) {
-  typedef Store<DT> S;
-  constexpr int QB = 4 * 16 * RW;
-  __shared__ uint4 kt_lds[KB * 8];  // [j][d]
-  __shared__ uint4 vt_lds[HD * 8];  // [d][j]
-
-  const int bh = blockIdx.y;
-  const int q0 = blockIdx.x * QB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, lg = lane >> 4;
-  const long N = long(B) * H * T;
-  const uint16_t *Qb = Q + long(bh) * T * HD;
-  const uint16_t *Vb = V + long(bh) * T * HD;
-  const int wrow0 = q0 + wave * 16 * RW;
-
-  // Q fragments (MFMA B operand): lane holds Q[i][8*(ks*4+lg) .. +8]
-  uint4 qf[RW][2];
-#pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    const int i = wrow0 + r * 16 + li;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      qf[r][ks] = (i < T) ? *reinterpret_cast<const uint4 *>(Qb + long(i) * HD + (ks * 4 + lg) * 8)
-                          : make_uint4(0, 0, 0, 0);
-    }
-  }
-
-  f32x4 o[RW][4];
-  float mrow[RW], lrow[RW];
-#pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    mrow[r] = -1e30f;
-    lrow[r] = 0.f;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) o[r][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  int kv_end = T;
-  if (causal) kv_end = min(T, q0 + QB);
-  const int ntiles = (kv_end + KB - 1) / KB;
-  const bool vec_ok = (T % 8) == 0;
-
-  for (int t = 0; t < ntiles; ++t) {
-    const int j0 = t * KB;
-    __syncthreads();  // previous tile fully consumed
-    // K slab: row d of the [hd, N] view holds 64 consecutive j at d*N+bh*T+j0
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int id = tid + it * 256, d = id >> 3, c = id & 7;
-      const int j = j0 + c * 8;
-      uint16_t vals[8];
-      const uint16_t *src = K + long(d) * N + long(bh) * T + j;
-      if (vec_ok && j + 8 <= T) {
-        uint4 v = *reinterpret_cast<const uint4 *>(src);
-        __builtin_memcpy(vals, &v, 16);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) vals[e] = (j + e < T) ? src[e] : uint16_t(0);
-      }
-      uint16_t *kl = reinterpret_cast<uint16_t *>(kt_lds);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int jj = c * 8 + e;
-        kl[swz(jj, d >> 3) * 8 + (d & 7)] = vals[e];
-      }
-    }
-    // V tile: rows j of [T, hd]; transposed into [d][j]
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int id = tid + it * 256, jj = id >> 3, c = id & 7;
-      const int j = j0 + jj;
-      uint4 v = (j < T) ? *reinterpret_cast<const uint4 *>(Vb + long(j) * HD + c * 8) : make_uint4(0, 0, 0, 0);
-      uint16_t vals[8];
-      __builtin_memcpy(vals, &v, 16);
-      uint16_t *vl = reinterpret_cast<uint16_t *>(vt_lds);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = c * 8 + e;
-        vl[swz(d, jj >> 3) * 8 + (jj & 7)] = vals[e];
-      }
-    }
-    __syncthreads();
-
-    if (causal && j0 > wrow0 + 16 * RW - 1) continue;  // whole wave masked
-
-    // ---- S^T = K * Q^T : lane holds S[i=li][j = jt*16 + 4*lg + e] ----
-    f32x4 s[RW][4];
-#pragma unroll
-    for (int r = 0; r < RW; ++r)
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt) s[r][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt) {
-        const uint4 kf = kt_lds[swz(jt * 16 + li, ks * 4 + lg)];
-#pragma unroll
-        for (int r = 0; r < RW; ++r) AttnMfma<DT>::mma(s[r][jt], kf, qf[r][ks]);
-      }
-    }
-
-    // ---- scale, mask, online softmax ----
-    uint4 pf[RW][2];
-#pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const int i = wrow0 + r * 16 + li;
-      float mx = -1e30f;
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int j = j0 + jt * 16 + lg * 4 + e;
-          float v = S::round(S::round(s[r][jt][e]) * scale);
-          const bool masked = (j >= T) || (causal && j > i);
-          v = masked ? -INFINITY : v;
-          s[r][jt][e] = v;
-          mx = fmaxf(mx, v);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mnew = fmaxf(mrow[r], mx);
-      const float alpha = __expf(mrow[r] - mnew);
-      mrow[r] = mnew;
-      float sum = 0.f;
-      uint16_t pb[4][4];
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float p = __expf(s[r][jt][e] - mnew);
-          sum += p;
-          pb[jt][e] = AttnMfma<DT>::cvt(p);
-        }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      lrow[r] = lrow[r] * alpha + sum;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) o[r][d] *= alpha;
-      // k-slot order for the PV step kk: j = 32kk + 4lg + {0..3}, 32kk + 16 + 4lg + {0..3}
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        uint16_t tmp[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          tmp[e] = pb[2 * kk][e];
-          tmp[4 + e] = pb[2 * kk + 1][e];
-        }
-        __builtin_memcpy(&pf[r][kk], tmp, 16);
-      }
-    }
-
-    // ---- O^T += V^T * P^T : lane holds O[i=li][d = dt*16 + 4*lg + e] ----
-    const uint16_t *vl = reinterpret_cast<const uint16_t *>(vt_lds);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const int d = dt * 16 + li;
-        const int ja = kk * 32 + lg * 4, jb = ja + 16;
-        const uint2 lo = *reinterpret_cast<const uint2 *>(vl + swz(d, ja >> 3) * 8 + (ja & 7));
-        const uint2 hi = *reinterpret_cast<const uint2 *>(vl + swz(d, jb >> 3) * 8 + (jb & 7));
-        const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
-#pragma unroll
-        for (int r = 0; r < RW; ++r) AttnMfma<DT>::mma(o[r][dt], vf, pf[r][kk]);
-      }
-    }
-  }
-
-  // ---- normalise, round, store merged [B, T, H*hd] ----
-  const int b = bh / H, h = bh - b * H;
-  const long E = long(H) * HD;
-#pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    const int i = wrow0 + r * 16 + li;
-    if (i >= T) continue;
-    const float inv = 1.0f / lrow[r];
-    uint16_t *dst = O + (long(b) * T + i) * E + long(h) * HD;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      u16x4 w;
-      w.x = S::enc(o[r][dt][0] * inv);
-      w.y = S::enc(o[r][dt][1] * inv);
-      w.z = S::enc(o[r][dt][2] * inv);
-      w.w = S::enc(o[r][dt][3] * inv);
-      *reinterpret_cast<u16x4 *>(dst + dt * 16 + lg * 4) = w;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// Main path (bf16/fp16, hd = 64, T % 8 == 0, power-of-two scale).
+// Single-trip flash kernel (bf16/fp16, hd % 8 == 0 up to 128, any T; MuNet's
+// or textbook keys).
 //
 // K and V tiles are staged in their natural layouts with 16-byte copies:
-//   K tile [d][j] : 64 rows of the [64, B*H*T] slab view, 64 columns each
-//   V tile [j][d] : 64 consecutive rows of the (b,h) block
+//   K tile [d][j] : the hd rows of the [hd, B*H*T] slab view, 64 columns each
+//   V tile [j][d] : 64 consecutive rows of the (b,h) block, as HDP / 64
+//                   sub-tiles of 64 columns
 // and the MFMA operands, which need 8 consecutive d (for K) or j (for V) per
 // lane, are read with ds_read_b64_tr_b16.  Within each group of 16 lanes that
 // instruction returns to lane i, element e, the value (i & 3) of the 8 bytes
@@ -305,12 +115,27 @@ flash_attn_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K
 // ((r >> SH) & 1)) (SH = 3 for K, 2 for V): the four rows one 16-lane group
 // reads and the rows of the neighbouring group land on disjoint banks.
 //
+// HDP is hd rounded up to 32, 64, 96 or 128: rows of K (and Q values) past hd
+// are zero, columns of O past hd are not stored.  The rows of MuNet's slab
+// start at any element (d N + bh T + j0), so K is loaded with 2-byte aligned
+// 16-byte loads; a tile's last chunk may read past column T (the masked
+// columns) but never past the end of K's buffer.
+//
+// RW: 16-row query groups per wave.  Each wave reads the whole K and V tile
+// from LDS, HDP * 256 bytes for RW * HDP / 4 + 2 RW MFMAs of 16 cycles: at
+// hd 128 one group needs 1024 LDS cycles per CU beside 544 MFMA cycles, two
+// groups break even, so hd > 64 takes RW = 2 while that leaves a workgroup
+// per CU.  A decoder block of 2 x 1000 tokens with 16 heads of 128: 1771 us
+// with the one-wave-per-query kernel that these sizes ran on, 310 us with this
+// one; a 237-token prompt at hd 64 (no 16-byte aligned K rows): 96 -> 88 us.
+//
 // Scores: the reference rounds q.k to the dtype and multiplies by the [1]
-// scale tensor (rounded again); with a power-of-two scale that product is
-// exact, so s = round(q.k) and the softmax runs in the log2 domain
-// u = s * scale * log2(e).  The running max is only raised when it grows by
-// more than 2^8 (p stays <= 256, exact enough for bf16 P and fp32 sums); row
-// sums stay lane-partial until the end.
+// scale tensor (rounded again).  With a power-of-two scale (P2: hd = 64) that
+// product is exact, so s = round(q.k) and the softmax runs in the log2 domain
+// u = s * scale * log2(e); else s = round(round(q.k) * scale) and u = s *
+// log2(e).  The running max is only raised when it grows by more than 2^8
+// (p stays <= 256, exact enough for bf16 P and fp32 sums); row sums stay
+// lane-partial until the end.
 typedef short v4s __attribute__((ext_vector_type(4)));
 
 template <int SH> __device__ __forceinline__ int tswz(int r, int c) {
@@ -325,24 +150,32 @@ __device__ __forceinline__ uint2 lds_tr(const uint8_t *p) {
 template <int V> struct BufIdx { static constexpr int value = V; };
 
 template <int DT> __device__ __forceinline__ void round_scores(float v[4]) {
-  if (DT == BF16) {
-    round4<BF16>(v);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = Store<F16>::round(v[e]);
-  }
+  round4<DT>(v);
+}
+
+// 16 bytes of 16-bit values from any element (the hardware takes global loads
+// of any alignment)
+typedef uint32_t v4u_any __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 ld16_any(const uint16_t *p) {
+  const v4u_any v = *reinterpret_cast<const v4u_any *>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
 }
 
 // TXT (textbook keys): K is head-split like V, key j of block bh at row
-// bh*T + j; its tile is staged in natural [j][d] layout (the swz pattern) and
-// the MFMA's K operand is read straight, without the transposing read.
-template <int DT, int RW, bool TXT>
-__global__ void __launch_bounds__(256)
+// bh*T + j; its tile is staged in natural [j][d] layout (the swz pattern, 64
+// columns per sub-tile) and the MFMA's K operand is read straight, without
+// the transposing read.
+template <int DT, int HDP, int RW, bool TXT, bool P2>
+__global__ void __launch_bounds__(256, 2)
 flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-                     uint16_t *__restrict__ O, int B, int H, int T, int causal, float c2) {
+                     uint16_t *__restrict__ O, int B, int H, int T, int hd, int causal, float scale, float c2) {
   constexpr int QB = 4 * 16 * RW;
+  constexpr int KS = HDP / 32, ND = HDP / 16, NSUB = (HDP + 63) / 64;
+  constexpr int NL = HDP / 32;   // 16-byte chunks each thread stages of a K or V tile
+  constexpr int VC = HDP / 8;    // chunks of a V row
   constexpr float kRaise = 8.0f;  // log2 of the largest unnormalised p
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][KB * HD * 2];  // [buf][K|V][tile]
+  constexpr int KBYTES = TXT ? NSUB * KB * 128 : HDP * 128, VBYTES = NSUB * KB * 128;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2][KBYTES + VBYTES];  // [buf][K | V tile]
 
   const int BH = B * H, nq = (T + QB - 1) / QB;
   const int lvl = blockIdx.x / BH, bh = blockIdx.x - lvl * BH;
@@ -350,38 +183,69 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const long N = long(BH) * T;
-  // column offset into the [64, N] slab, or the block's first key row (TXT)
-  const uint16_t *Kb = TXT ? K + long(bh) * T * HD : K + long(bh) * T;
-  const uint16_t *Vb = V + long(bh) * T * HD;
+  // column offset into the [hd, N] slab, or the block's first key row (TXT)
+  const uint16_t *Kb = TXT ? K + long(bh) * T * hd : K + long(bh) * T;
+  const uint16_t *Vb = V + long(bh) * T * hd;
   const int wrow0 = q0 + wave * 16 * RW;
 
   // rows past T (ragged last block) read row T-1; their results are not stored
-  uint4 qf[RW][2];
+  uint4 qf[RW][KS];
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
     const int i = min(wrow0 + r * 16 + li, T - 1);
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      qf[r][ks] = *reinterpret_cast<const uint4 *>(Q + (long(bh) * T + i) * HD + ks * 32 + lg * 8);
+    for (int ks = 0; ks < KS; ++ks) {
+      const int d = ks * 32 + lg * 8;
+      qf[r][ks] = d < hd ? *reinterpret_cast<const uint4 *>(Q + (long(bh) * T + i) * hd + d) : make_uint4(0, 0, 0, 0);
+    }
   }
   // o: lane holds O[i = li][d = dt*16 + 4*lg + e]; osum: the row sum of the
   // (rounded) P fed to the MFMA, from a ones operand; mrow: running max (log2 units)
-  f32x4 o[RW][4], osum[RW];
+  f32x4 o[RW][ND], osum[RW];
   float mrow[RW];
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
-    mrow[r] = -1e30f;
+    mrow[r] = -3.4028234e38f;  // below every finite score
     osum[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int d = 0; d < 4; ++d) o[r][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < ND; ++d) o[r][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const uint32_t one2 = DT == BF16 ? 0x3F803F80u : 0x3C003C00u;
   const uint4 ones = make_uint4(one2, one2, one2, one2);
 
-  // staging: rows r0 and r0 + 32 of each tile, chunk c0
-  const int r0 = tid >> 3, c0 = tid & 7;
-  const int st_k0 = (TXT ? swz(r0, c0) : tswz<3>(r0, c0)) * 16, st_k1 = (TXT ? swz(r0 + 32, c0) : tswz<3>(r0 + 32, c0)) * 16;
-  const int st_v0 = tswz<2>(r0, c0) * 16, st_v1 = tswz<2>(r0 + 32, c0) * 16;
+  // staging.  K (MuNet): chunk kc of rows kr0 + 32i; V (and K, TXT): chunk
+  // id % VC of row id / VC, id = tid + 256 i.  Chunks past hd (kin / vin
+  // false) load from inside the tensor and are not stored.
+  const int kr0 = tid >> 3, kc = tid & 7;
+  const uint16_t *kp[NL], *vp[NL];
+  int kst[NL], vst[NL], vrow[NL];
+  bool kin[NL], vin[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int id = tid + 256 * i, row = id / VC, c = id % VC;
+    vrow[i] = row;
+    vin[i] = c * 8 < hd;
+    const long voff = long(row) * hd + (vin[i] ? c * 8 : 0);
+    vp[i] = Vb + voff;
+    vst[i] = KBYTES + (c >> 3) * (KB * 128) + tswz<2>(row, c & 7) * 16;
+    if constexpr (TXT) {
+      kin[i] = vin[i];
+      kp[i] = Kb + voff;
+      kst[i] = (c >> 3) * (KB * 128) + swz(row, c & 7) * 16;
+    } else {
+      const int d = kr0 + 32 * i;
+      kin[i] = d < hd;
+      kp[i] = Kb + long(min(d, hd - 1)) * N + kc * 8;
+      kst[i] = tswz<3>(d, kc) * 16;
+    }
+  }
+  // K rows / chunks past hd are zero in both buffers
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+    if (!kin[i]) {
+      *reinterpret_cast<uint4 *>(&lds[0][kst[i]]) = make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4 *>(&lds[1][kst[i]]) = make_uint4(0, 0, 0, 0);
+    }
   // transposed reads: this lane addresses row base + (s >> 2), 8 bytes at
   // column 4(s & 3) of a 16-column block; the row swizzle term is lane-fixed
   const int s16 = lane & 15, sr = s16 >> 2, sx = ((s16 & 3) >> 1) ^ (2 * (sr ^ (lg & 1))), sh = (s16 & 1) * 8;
@@ -392,38 +256,48 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
   const int ntiles = (kv_end + KB - 1) / KB;
   // loop-carried load pointers (advanced one tile per gload) keep the address
   // registers live, so they are never recycled while a prefetch is in flight
-  const long kld = TXT ? HD : N;  // elements between the rows of a K tile
-  const uint16_t *kp0 = Kb + long(r0) * kld + c0 * 8, *kp1 = Kb + long(r0 + 32) * kld + c0 * 8;
-  const uint16_t *vp0 = Vb + long(r0) * HD + c0 * 8, *vp1 = Vb + long(r0 + 32) * HD + c0 * 8;
-  uint4 kr[2], vr[2];
+  const long kstep = TXT ? long(KB) * hd : KB, vstep = long(KB) * hd;
+  const uint16_t *kend = K + N * hd;  // end of K's buffer
+  uint4 kr[NL], vr[NL];
   auto gload = [&](int j0) {
     if (j0 + KB <= T) {  // whole tile in range (wave-uniform)
-      kr[0] = *reinterpret_cast<const uint4 *>(kp0);
-      kr[1] = *reinterpret_cast<const uint4 *>(kp1);
-      vr[0] = *reinterpret_cast<const uint4 *>(vp0);
-      vr[1] = *reinterpret_cast<const uint4 *>(vp1);
-    } else if (TXT) {  // ragged last tile: zero the rows past T
-      kr[0] = (j0 + r0 < T) ? *reinterpret_cast<const uint4 *>(kp0) : make_uint4(0, 0, 0, 0);
-      kr[1] = (j0 + r0 + 32 < T) ? *reinterpret_cast<const uint4 *>(kp1) : make_uint4(0, 0, 0, 0);
-      vr[0] = (j0 + r0 < T) ? *reinterpret_cast<const uint4 *>(vp0) : make_uint4(0, 0, 0, 0);
-      vr[1] = (j0 + r0 + 32 < T) ? *reinterpret_cast<const uint4 *>(vp1) : make_uint4(0, 0, 0, 0);
-    } else {  // ragged last tile: zero what lies past T
-      const bool kin = j0 + c0 * 8 < T;
-      kr[0] = kin ? *reinterpret_cast<const uint4 *>(kp0) : make_uint4(0, 0, 0, 0);
-      kr[1] = kin ? *reinterpret_cast<const uint4 *>(kp1) : make_uint4(0, 0, 0, 0);
-      vr[0] = (j0 + r0 < T) ? *reinterpret_cast<const uint4 *>(vp0) : make_uint4(0, 0, 0, 0);
-      vr[1] = (j0 + r0 + 32 < T) ? *reinterpret_cast<const uint4 *>(vp1) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < NL; ++i) kr[i] = TXT ? *reinterpret_cast<const uint4 *>(kp[i]) : ld16_any(kp[i]);
+#pragma unroll
+      for (int i = 0; i < NL; ++i) vr[i] = *reinterpret_cast<const uint4 *>(vp[i]);
+    } else {
+      // ragged last tile: V (and textbook K) rows past T are zero; MuNet's K
+      // columns past T are masked after the product, so they may hold
+      // whatever follows, up to the buffer's last element
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const bool in = j0 + vrow[i] < T;
+        vr[i] = in ? *reinterpret_cast<const uint4 *>(vp[i]) : make_uint4(0, 0, 0, 0);
+        if constexpr (TXT) {
+          kr[i] = in ? *reinterpret_cast<const uint4 *>(kp[i]) : make_uint4(0, 0, 0, 0);
+        } else if (kend - kp[i] >= 8) {
+          kr[i] = ld16_any(kp[i]);
+        } else {
+          uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (kend - kp[i] > e) w[e >> 1] |= uint32_t(kp[i][e]) << (16 * (e & 1));
+          kr[i] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+      }
     }
-    kp0 += TXT ? KB * HD : KB;
-    kp1 += TXT ? KB * HD : KB;
-    vp0 += KB * HD;
-    vp1 += KB * HD;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      kp[i] += kstep;
+      vp[i] += vstep;
+    }
   };
   auto sstore = [&](int buf) {
-    *reinterpret_cast<uint4 *>(&lds[buf][0][st_k0]) = kr[0];
-    *reinterpret_cast<uint4 *>(&lds[buf][0][st_k1]) = kr[1];
-    *reinterpret_cast<uint4 *>(&lds[buf][1][st_v0]) = vr[0];
-    *reinterpret_cast<uint4 *>(&lds[buf][1][st_v1]) = vr[1];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      if (kin[i]) *reinterpret_cast<uint4 *>(&lds[buf][kst[i]]) = kr[i];
+      if (vin[i]) *reinterpret_cast<uint4 *>(&lds[buf][vst[i]]) = vr[i];
+    }
   };
   if (ntiles > 0) {
     gload(0);
@@ -436,7 +310,7 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
 #pragma unroll
   for (int r = 0; r < RW; ++r)
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
       asm volatile("" : "+v"(qf[r][ks].x), "+v"(qf[r][ks].y), "+v"(qf[r][ks].z), "+v"(qf[r][ks].w)::"memory");
 
   // one K/V tile; the LDS buffer index is a compile-time constant (the loop
@@ -448,30 +322,30 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
     if (t + 1 < ntiles) gload(j0 + KB);
 
     if (!(causal && j0 > wrow0 + 16 * RW - 1)) {  // skip tiles wholly above the diagonal
-      const uint8_t *kt = lds[buf][0], *vt = lds[buf][1];
+      const uint8_t *kt = lds[buf], *vt = lds[buf] + KBYTES;
       // ---- S^T = K * Q^T : lane holds S[i = li][j = jt*16 + 4*lg + e] ----
-      uint4 kf[2][4];
+      f32x4 s[RW][4];
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
+      for (int jt = 0; jt < 4; ++jt) {
+        uint4 kf[KS];
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
+        for (int ks = 0; ks < KS; ++ks) {
           if constexpr (TXT) {
-            kf[ks][jt] = *reinterpret_cast<const uint4 *>(kt + swz(jt * 16 + li, ks * 4 + lg) * 16);
+            const int c = ks * 4 + lg;
+            kf[ks] = *reinterpret_cast<const uint4 *>(kt + (ks >> 1) * (KB * 128) + swz(jt * 16 + li, c & 7) * 16);
           } else {
             const uint8_t *p = kt + rd_k + ((2 * jt) ^ sx) * 16 + ks * 32 * 128;
             const uint2 lo = lds_tr(p), hi = lds_tr(p + 4 * 128);
-            kf[ks][jt] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            kf[ks] = make_uint4(lo.x, lo.y, hi.x, hi.y);
           }
         }
-      f32x4 s[RW][4];
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt)
+        for (int r = 0; r < RW; ++r) s[r][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < RW; ++r) {
-          s[r][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-          AttnMfma<DT>::mma(s[r][jt], kf[0][jt], qf[r][0]);
-          AttnMfma<DT>::mma(s[r][jt], kf[1][jt], qf[r][1]);
-        }
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int r = 0; r < RW; ++r) AttnMfma<DT>::mma(s[r][jt], kf[ks], qf[r][ks]);
+      }
 
       uint4 pf[RW][2];
 #pragma unroll
@@ -481,6 +355,11 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
         for (int jt = 0; jt < 4; ++jt) {
           float w[4] = {s[r][jt][0], s[r][jt][1], s[r][jt][2], s[r][jt][3]};
           round_scores<DT>(w);
+          if constexpr (!P2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] *= scale;
+            round_scores<DT>(w);
+          }
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[jt * 4 + e] = w[e];
         }
@@ -506,7 +385,7 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
           mrow[r] = mnew;
           osum[r] *= alpha;
 #pragma unroll
-          for (int d = 0; d < 4; ++d) o[r][d] *= alpha;
+          for (int d = 0; d < ND; ++d) o[r][d] *= alpha;
         }
         const float nm = -mrow[r];
         uint32_t pk[8];
@@ -522,18 +401,15 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
       // ---- O^T += V^T * P^T : lane holds O[i = li][d = dt*16 + 4*lg + e] ----
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        uint4 vf[4];
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const uint8_t *p = vt + rd_v + ((2 * dt) ^ sx) * 16 + kk * 32 * 128;
+        for (int r = 0; r < RW; ++r) AttnMfma<DT>::mma(osum[r], ones, pf[r][kk]);
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) {
+          const uint8_t *p = vt + (dt >> 2) * (KB * 128) + rd_v + ((2 * (dt & 3)) ^ sx) * 16 + kk * 32 * 128;
           const uint2 lo = lds_tr(p), hi = lds_tr(p + 16 * 128);
-          vf[dt] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-        }
+          const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
 #pragma unroll
-        for (int r = 0; r < RW; ++r) {
-          AttnMfma<DT>::mma(osum[r], ones, pf[r][kk]);
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) AttnMfma<DT>::mma(o[r][dt], vf[dt], pf[r][kk]);
+          for (int r = 0; r < RW; ++r) AttnMfma<DT>::mma(o[r][dt], vf, pf[r][kk]);
         }
       }
     }
@@ -548,15 +424,16 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
   if (t < ntiles) tile(t, BufIdx<0>{});
 
   const int b = bh / H, h = bh - b * H;
-  const long E = long(H) * HD;
+  const long E = long(H) * hd;
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
     const int i = wrow0 + r * 16 + li;
     if (i >= T) continue;
     const float inv = 1.0f / osum[r][0];
-    uint16_t *dst = O + (long(b) * T + i) * E + long(h) * HD;
+    uint16_t *dst = O + (long(b) * T + i) * E + long(h) * hd;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
+    for (int dt = 0; dt < ND; ++dt) {
+      if (dt * 16 + lg * 4 >= hd) continue;
       u16x4 w;
       w.x = Store<DT>::enc(o[r][dt][0] * inv);
       w.y = Store<DT>::enc(o[r][dt][1] * inv);
@@ -911,6 +788,45 @@ int cu_count() {
   }
   return cached[dev] > 0 ? cached[dev] : 0;
 }
+// flash_attn_tr_kernel for this head size: one 16-row query group per wave
+// (more resident waves hide the softmax latency) up to hd 64; above, two
+// groups per wave, whose shared fragment reads balance LDS against the matrix
+// cores, once that still gives every CU a workgroup.
+template <int DT>
+hipError_t flash_tr(const void *q, const void *k, const void *v, void *ctx, int B, int H, int T, int hd, int causal,
+                    float scale, int textbook, hipStream_t st) {
+  const uint16_t *Q = (const uint16_t *)q, *K = (const uint16_t *)k, *V = (const uint16_t *)v;
+  uint16_t *O = (uint16_t *)ctx;
+  const long bh = long(B) * H;
+  const bool p2 = hd == HD && pow2(scale);
+  static const int forced = tr_rows_env();
+  const int rw = hd <= 64 ? (forced && p2 && !textbook ? forced : 1) : long((T + 127) / 128) * bh >= 256 ? 2 : 1;
+  const dim3 grid(unsigned(long((T + 64 * rw - 1) / (64 * rw)) * bh));
+  const float c2 = (p2 ? scale : 1.0f) * 1.4426950408889634f;
+#define MH_TR(HDP, RW, TXT, P2)                                                                                    \
+  hipLaunchKernelGGL((flash_attn_tr_kernel<DT, HDP, RW, TXT, P2>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, hd, \
+                     causal, scale, c2)
+#define MH_TR_RW(HDP) \
+  { if (rw == 2) { if (textbook) MH_TR(HDP, 2, true, false); else MH_TR(HDP, 2, false, false); } \
+    else { if (textbook) MH_TR(HDP, 1, true, false); else MH_TR(HDP, 1, false, false); } }
+  if (p2) {
+    if (textbook) MH_TR(64, 1, true, true);
+    else if (rw == 2) MH_TR(64, 2, false, true);
+    else MH_TR(64, 1, false, true);
+  } else if (hd <= 32) {
+    if (textbook) MH_TR(32, 1, true, false); else MH_TR(32, 1, false, false);
+  } else if (hd <= 64) {
+    if (textbook) MH_TR(64, 1, true, false); else MH_TR(64, 1, false, false);
+  } else if (hd <= 96) {
+    MH_TR_RW(96)
+  } else {
+    MH_TR_RW(128)
+  }
+#undef MH_TR_RW
+#undef MH_TR
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t attention(int dt, const void *q, const void *k, const void *v, void *ctx, int B, int H, int T, int hd,
@@ -918,17 +834,6 @@ hipError_t attention(int dt, const void *q, const void *k, const void *v, void *
   if (B <= 0 || H <= 0 || T <= 0) return hipSuccess;
   const bool aligned = ((uintptr_t)q % 16 == 0) && ((uintptr_t)k % 16 == 0) && ((uintptr_t)v % 16 == 0) &&
                        ((uintptr_t)ctx % 8 == 0);
-  if (textbook && !force_generic && hd == HD && (dt == BF16 || dt == F16) && aligned && pow2(scale)) {
-    // textbook keys: rows of K like V, so any T (ragged tiles are row-masked)
-    const int bh = B * H;
-    const dim3 grid(unsigned(long((T + 63) / 64) * bh));
-    const float c2 = scale * 1.4426950408889634f;
-    const uint16_t *Q = (const uint16_t *)q, *K = (const uint16_t *)k, *V = (const uint16_t *)v;
-    uint16_t *O = (uint16_t *)ctx;
-    if (dt == BF16) hipLaunchKernelGGL((flash_attn_tr_kernel<BF16, 1, true>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2);
-    else hipLaunchKernelGGL((flash_attn_tr_kernel<F16, 1, true>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2);
-    return hipGetLastError();
-  }
   const bool use_pipe = pipe_kernel_env();
   if (use_pipe && !textbook && !force_generic && hd == HD && (dt == BF16 || dt == F16) && aligned && T % KB == 0 &&
       pow2(scale)) {
@@ -946,43 +851,14 @@ hipError_t attention(int dt, const void *q, const void *k, const void *v, void *
       hipLaunchKernelGGL((flash_attn_pipe_kernel<F16>), dim3(unsigned(items)), dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2, snake);
     return hipGetLastError();
   }
-  if (!textbook && !force_generic && hd == HD && (dt == BF16 || dt == F16) && aligned && T % 8 == 0 && pow2(scale)) {
-    const int bh = B * H;
-    static const int forced = tr_rows_env();
-    // 16 query rows per wave: more resident waves hide the softmax latency
-    // better than the operand reuse of 32 rows per wave (measured on MI355X)
-    const int rw = forced ? forced : 1;
-    const int qb = 64 * rw;
-    const dim3 grid(unsigned(long((T + qb - 1) / qb) * bh));
-    const float c2 = scale * 1.4426950408889634f;
-    const uint16_t *Q = (const uint16_t *)q, *K = (const uint16_t *)k, *V = (const uint16_t *)v;
-    uint16_t *O = (uint16_t *)ctx;
-    if (dt == BF16) {
-      if (rw == 2) hipLaunchKernelGGL((flash_attn_tr_kernel<BF16, 2, false>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2);
-      else hipLaunchKernelGGL((flash_attn_tr_kernel<BF16, 1, false>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2);
-    } else {
-      if (rw == 2) hipLaunchKernelGGL((flash_attn_tr_kernel<F16, 2, false>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2);
-      else hipLaunchKernelGGL((flash_attn_tr_kernel<F16, 1, false>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2);
-    }
-    return hipGetLastError();
+  if (!force_generic && (dt == BF16 || dt == F16) && aligned && hd % 8 == 0 && hd <= 128) {
+    if (long((T + 63) / 64) * B * H > 0x7fffffffL) return hipErrorInvalidValue;
+    return dt == BF16 ? flash_tr<BF16>(q, k, v, ctx, B, H, T, hd, causal, scale, textbook, st)
+                      : flash_tr<F16>(q, k, v, ctx, B, H, T, hd, causal, scale, textbook, st);
   }
-  if (!textbook && !force_generic && hd == HD && (dt == BF16 || dt == F16) && aligned) {
-    const int bh = B * H;
-    // 128-row blocks when that still fills the chip, else 64-row blocks
-    const int rw = (long((T + 127) / 128) * bh >= 512) ? 2 : 1;
-    const int qb = 64 * rw;
-    dim3 grid((T + qb - 1) / qb, bh);
-    const uint16_t *Q = (const uint16_t *)q, *K = (const uint16_t *)k, *V = (const uint16_t *)v;
-    uint16_t *O = (uint16_t *)ctx;
-    if (dt == BF16) {
-      if (rw == 2) hipLaunchKernelGGL((flash_attn_kernel<BF16, 2>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, scale);
-      else hipLaunchKernelGGL((flash_attn_kernel<BF16, 1>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, scale);
-    } else {
-      if (rw == 2) hipLaunchKernelGGL((flash_attn_kernel<F16, 2>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, scale);
-      else hipLaunchKernelGGL((flash_attn_kernel<F16, 1>), grid, dim3(256), 0, st, Q, K, V, O, B, H, T, causal, scale);
-    }
-    return hipGetLastError();
-  }
+  if (!force_generic && dt == F32 && aligned && attention_f32_ok(hd, ctx))
+    return attention_f32((const float *)q, (const float *)k, (const float *)v, (float *)ctx, B, H, T, hd, causal, scale,
+                         textbook, st);
   if (size_t(T) * 4 > 64 * 1024) return hipErrorInvalidValue;
   dim3 grid(T, B * H);
   const size_t lds = size_t(T) * 4;

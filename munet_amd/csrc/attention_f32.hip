@@ -1,0 +1,274 @@
+// fp32 fused attention for gfx950 (the fp32 case of attention.hip: the core
+// of nn::MultiHeadAttention, reference src/nn/attention.hpp:51-99, with
+// MuNet's reading of k's buffer as a [hd, B*H*T] matrix, or textbook keys).
+//
+// Flash form on v_mfma_f32_16x16x4f32 (full fp32 products and sums): one
+// workgroup of four waves per 64 queries of a (b, h) block, 64 keys per tile,
+// each wave 16 queries.  S^T = K Q^T and O^T = V^T P^T, so every lane owns
+// one query (its column of both products) and P goes from the S accumulators
+// into the PV operand register for register.
+//
+// The matrix rows are spread over the lanes so that every LDS read is 16
+// bytes and feeds four (PV: CW) MFMAs:
+//   * k-slot lg of step (ks, e) of QK holds d = 16 ks + 4 lg + e;
+//   * MuNet's K tile is [d][j]: row li of product x is key 4 li + x, so one
+//     read of K[d][4 li ..] serves x = 0..3, and lane (li, lg) ends with keys
+//     16 lg + 4 e + x of query li in s[x][e].  A textbook tile is [j][d]: one
+//     read of K[16 x + li][16 ks + 4 lg ..] serves e = 0..3, and s[x][e] is
+//     key 16 x + 4 lg + e;
+//   * PV step (x, e) takes s[x][e] as it is: its k-slot lg is that key; row li
+//     of product (g, w) is column CW (16 g + li) + w, so one read of CW floats
+//     of V's row serves w = 0..CW-1 and each lane stores CW consecutive floats.
+// HDP = 16 NG CW is hd rounded up to 32, 64, 96 or 128; Q and K past hd are
+// zero.  A ragged last tile's K columns may hold what follows in the buffer
+// (masked after the product); V rows past T are zero.
+//
+// The work is bound by the fp32 matrix rate (64 keys x 16 queries x hd 64:
+// 128 MFMAs of 32 cycles beside about 250 VALU instructions), so the tiles
+// are single-buffered in LDS with the next tile in registers: 32 KB at hd 64
+// leaves room for several workgroups per CU.  Encoder layer of 8 x 250 tokens,
+// 8 heads of 64: the block took 382 us with the one-wave-per-query kernel that
+// this replaces, 215 us with this one, at the same error against float64.
+//
+// Precision: exp(v - m) with m the exact running row max, its base-2 argument
+// carried in two floats (the one-float product loses |v - m| 2^-24).
+#include "mh_common.hpp"
+#include "mh_kernels.hpp"
+
+namespace mh {
+namespace {
+
+constexpr int KB = 64;
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// exp(x) for x <= 0 (-inf gives 0, NaN stays NaN): 2^(hi + lo) with x log2(e)
+// = hi + lo
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float kL = 1.44269502162933349609375f, kLlo = 1.92596303e-8f, kLn2 = 0.693147181f;
+  x = x < -200.f ? -200.f : x;
+  const float hi = __fmul_rn(x, kL);
+  const float lo = __fmaf_rn(x, kLlo, __fmaf_rn(x, kL, -hi));
+  const float p = __builtin_amdgcn_exp2f(hi);
+  return __fmaf_rn(p, __fmul_rn(lo, kLn2), p);
+}
+
+template <int NG, int CW, bool TXT>
+__global__ void __launch_bounds__(256)
+flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
+                      float *__restrict__ O, int B, int H, int T, int hd, int causal, float scale) {
+  constexpr int HDP = NG * 16 * CW, KS = HDP / 16, VC = HDP / 4;  // VC: 16-byte chunks of a V row
+  constexpr int NL = HDP / 16;                                     // chunks each thread stages of a K or V tile
+  typedef float vcw __attribute__((ext_vector_type(CW)));
+  __shared__ __attribute__((aligned(16))) float ks_[64 * HDP], vs_[64 * HDP];
+
+  const int BH = B * H, nq = (T + KB - 1) / KB;
+  const int lvl = blockIdx.x / BH, bh = blockIdx.x - lvl * BH;
+  const int q0 = (causal ? nq - 1 - lvl : lvl) * KB;  // causal: longest rows first
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const long N = long(BH) * T;
+  const float *Kb = TXT ? K + long(bh) * T * hd : K + long(bh) * T;
+  const float *Vb = V + long(bh) * T * hd;
+  const float *kend = K + N * hd;
+  const int wrow0 = q0 + wave * 16, i = wrow0 + li;
+
+  f32x4 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d = 16 * ks + 4 * lg;
+    qf[ks] = d < hd ? *reinterpret_cast<const f32x4 *>(Q + (long(bh) * T + min(i, T - 1)) * hd + d)
+                    : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  f32x4 o[NG][CW];
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int w = 0; w < CW; ++w) o[g][w] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -3.4028234e38f, l = 0.f;
+
+  // staging: chunk id = tid + 256 n of a tile
+  const float *kp[NL], *vp[NL];
+  int kst[NL], vst[NL], vrow[NL];
+  bool kin[NL], vin[NL];
+#pragma unroll
+  for (int n = 0; n < NL; ++n) {
+    const int id = tid + 256 * n, row = id / VC, c = id % VC;
+    vrow[n] = row;
+    vin[n] = 4 * c < hd;
+    const long voff = long(row) * hd + (vin[n] ? 4 * c : 0);
+    vp[n] = Vb + voff;
+    vst[n] = row * HDP + 4 * c;
+    if constexpr (TXT) {
+      kin[n] = vin[n];
+      kp[n] = Kb + voff;
+      kst[n] = row * HDP + 4 * (c ^ (row & 7));
+    } else {
+      const int d = id >> 4;
+      kin[n] = d < hd;
+      kp[n] = Kb + long(min(d, hd - 1)) * N + 4 * (id & 15);
+      kst[n] = d * KB + 4 * (id & 15);
+    }
+    if (!kin[n]) *reinterpret_cast<f32x4 *>(ks_ + kst[n]) = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const long kstep = TXT ? long(KB) * hd : KB, vstep = long(KB) * hd;
+  f32x4 kr[NL], vr[NL];
+  auto gload = [&](int j0) {
+    if (j0 + KB <= T) {
+#pragma unroll
+      for (int n = 0; n < NL; ++n) {
+        if constexpr (TXT) kr[n] = *reinterpret_cast<const f32x4 *>(kp[n]);
+        else kr[n] = *reinterpret_cast<const f32x4_any *>(kp[n]);
+        vr[n] = *reinterpret_cast<const f32x4 *>(vp[n]);
+      }
+    } else {
+#pragma unroll
+      for (int n = 0; n < NL; ++n) {
+        const bool in = j0 + vrow[n] < T;
+        const f32x4 vv = *reinterpret_cast<const f32x4 *>(in ? vp[n] : Vb);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vr[n][e] = in ? vv[e] : 0.f;
+        if constexpr (TXT) {
+          const f32x4 kv = *reinterpret_cast<const f32x4 *>(in ? kp[n] : Kb);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) kr[n][e] = in ? kv[e] : 0.f;
+        } else if (kend - kp[n] >= 4) {
+          kr[n] = *reinterpret_cast<const f32x4_any *>(kp[n]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) kr[n][e] = kend - kp[n] > e ? kp[n][e] : 0.f;
+        }
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      kp[n] += kstep;
+      vp[n] += vstep;
+    }
+  };
+
+  const int kv_end = causal ? min(T, q0 + KB) : T;
+  const int ntiles = (kv_end + KB - 1) / KB;
+  gload(0);
+  for (int t = 0; t < ntiles; ++t) {
+    const int j0 = t * KB;
+    __syncthreads();  // the previous tile has been read
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      if (kin[n]) *reinterpret_cast<f32x4 *>(ks_ + kst[n]) = kr[n];
+      if (vin[n]) *reinterpret_cast<f32x4 *>(vs_ + vst[n]) = vr[n];
+    }
+    __syncthreads();
+    if (t + 1 < ntiles) gload(j0 + KB);
+
+    f32x4 s[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) s[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (TXT) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        f32x4 kf[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          kf[x] = *reinterpret_cast<const f32x4 *>(ks_ + (16 * x + li) * HDP + 4 * ((4 * ks + lg) ^ (li & 7)));
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) s[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[x][e], qf[ks][e], s[x], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x4 kf = *reinterpret_cast<const f32x4 *>(ks_ + (16 * ks + 4 * lg + e) * KB + 4 * li);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) s[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[x], qf[ks][e], s[x], 0, 0, 0);
+        }
+    }
+
+    const bool edge = j0 + KB > T || (causal && j0 + KB - 1 > wrow0);  // wave-uniform
+    const int lim = (causal ? min(T - 1, i) : T - 1) - j0;             // last unmasked key of this query
+    float mx = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = __fmul_rn(s[x][e], scale);
+        if (edge && (TXT ? 16 * x + 4 * lg + e : 16 * lg + 4 * e + x) > lim) v = -INFINITY;
+        s[x][e] = v;
+        mx = fmaxf(mx, v);
+      }
+    mx = xor32_max(xor16_max(mx));
+    if (__any(mx > m)) {
+      const float mnew = fmaxf(m, mx), alpha = exp_neg(m - mnew);
+      m = mnew;
+      l *= alpha;
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int w = 0; w < CW; ++w) o[g][w] *= alpha;
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[x][e] = exp_neg(s[x][e] - m);
+        l += s[x][e];
+      }
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = TXT ? 16 * x + 4 * lg + e : 16 * lg + 4 * e + x;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          const vcw vf = *reinterpret_cast<const vcw *>(vs_ + row * HDP + CW * (16 * g + li));
+#pragma unroll
+          for (int w = 0; w < CW; ++w) o[g][w] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[w], s[x][e], o[g][w], 0, 0, 0);
+        }
+      }
+  }
+
+  l = xor32_add(xor16_add(l));
+  if (i >= T) return;
+  const int b = bh / H, h = bh - b * H;
+  float *dst = O + (long(b) * T + i) * (long(H) * hd) + long(h) * hd;
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = CW * (16 * g + 4 * lg + e);
+      if (d >= hd) continue;
+      vcw w4;
+#pragma unroll
+      for (int w = 0; w < CW; ++w) w4[w] = o[g][w][e] / l;
+      *reinterpret_cast<vcw *>(dst + d) = w4;
+    }
+}
+
+}  // namespace
+
+bool attention_f32_ok(int hd, const void *ctx) { return hd > 0 && hd <= 128 && hd % 4 == 0 && (uintptr_t)ctx % 16 == 0; }
+
+hipError_t attention_f32(const float *q, const float *k, const float *v, float *ctx, int B, int H, int T, int hd,
+                         int causal, float scale, int textbook, hipStream_t st) {
+  const long items = long((T + KB - 1) / KB) * B * H;
+  if (items > 0x7fffffffL || !attention_f32_ok(hd, ctx)) return hipErrorInvalidValue;
+  const dim3 grid{unsigned(items)};
+#define MH_AF(NG, CW)                                                                                             \
+  {                                                                                                               \
+    if (textbook) hipLaunchKernelGGL((flash_attn_f32_kernel<NG, CW, true>), grid, dim3(256), 0, st, q, k, v, ctx, \
+                                     B, H, T, hd, causal, scale);                                                 \
+    else hipLaunchKernelGGL((flash_attn_f32_kernel<NG, CW, false>), grid, dim3(256), 0, st, q, k, v, ctx, B, H,   \
+                            T, hd, causal, scale);                                                                \
+  }
+  if (hd <= 32) MH_AF(1, 2)
+  else if (hd <= 64) MH_AF(1, 4)
+  else if (hd <= 96) MH_AF(3, 2)
+  else MH_AF(2, 4)
+#undef MH_AF
+  return hipGetLastError();
+}
+
+}  // namespace mh

@@ -156,6 +156,12 @@ hipError_t gemm_splitk(int dt, const void *A, const void *Bt, int M, int N, int 
 hipError_t attention(int dt, const void *q, const void *k, const void *v, void *ctx, int B, int H, int T, int hd,
                      int causal, float scale, int force_generic, hipStream_t st, int textbook = 0);
 
+// fp32 flash attention (attention_f32.hip): hd <= 128, hd % 4 == 0, every
+// pointer 16-byte aligned.
+bool attention_f32_ok(int hd, const void *ctx);
+hipError_t attention_f32(const float *q, const float *k, const float *v, float *ctx, int B, int H, int T, int hd,
+                         int causal, float scale, int textbook, hipStream_t st);
+
 // KV-cache decode (decode.hip).  state: device ints {pos, step, pending}:
 // the position of the tokens being fed, the index of the next generated
 // token in `tokens`, and 1 while the head's greedy choices in best still have

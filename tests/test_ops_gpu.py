@@ -128,10 +128,10 @@ def test_qkv_headsplit_bits(hip, dt, B, T, E, H):
 @pytest.mark.parametrize("causal", [False, True])
 def test_attention_core(hip, orc, dt, B, T, H, hd, causal):
     """q/k/v projection (fused head split) + fused attention vs the reference
-    MHA core, including MuNet's K-reinterpretation.  hd = 64 with T % 8 == 0
-    runs the pre-transposed-operand kernel (T = 72 with 256 (b,h) blocks takes
-    its 32-rows-per-wave variant and a ragged last tile); T = 77 runs the
-    in-LDS-transpose kernel; the rest the generic kernel."""
+    MHA core, including MuNet's K-reinterpretation.  hd = 64 with T % 64 == 0
+    runs the software-pipelined kernel, the other multiples of 8 the
+    single-trip flash kernel (T = 72 and 77 with a ragged last tile), hd 4 the
+    generic kernel in the 16-bit types."""
     E = H * hd
     x = rand((B * T, E), dt, 20)
     p = _mha_params(E, dt, 30)
@@ -150,6 +150,49 @@ def test_attention_core(hip, orc, dt, B, T, H, hd, causal):
     ctx = empty((B * T, E), dt)
     hip.attention(q, k, v, ctx, B, H, T, hd, causal)
     assert_close(to_host(ctx, dt), ref, dt, what="attention")
+
+
+@pytest.mark.parametrize("dt", [F16, BF16, F32])
+@pytest.mark.parametrize("hd", [8, 16, 32, 40, 48, 64, 80, 96, 104, 128, 20])
+@pytest.mark.parametrize("B,H,T", [(1, 1, 1), (1, 2, 7), (2, 1, 63), (1, 2, 65), (1, 1, 130), (2, 130, 33)])
+@pytest.mark.parametrize("causal,textbook", [(False, False), (True, False), (True, True), (False, True)])
+def test_attention_head_sizes(hip, dt, hd, B, H, T, causal, textbook):
+    """The flash kernels over head sizes (each rounded size 32 / 64 / 96 / 128,
+    its edges and its padding; hd 20 is the 16-bit generic kernel), ragged
+    lengths around the 64-key tile, rows of MuNet's key matrix that start at
+    any alignment, one and two query groups per wave ((2, 130, 33) has 260
+    workgroups), and a key buffer whose last chunk ends at the allocation's
+    end.  Oracle: float64 attention with the reference's score roundings.
+
+    Tolerances, against rows of max |ctx| about 1: fp32 2e-5, the scores' sum
+    error (hd 2^-24 |q||k| scale, about 1e-6) plus T sums; 16-bit: 2^-8 (bf16)
+    and 2^-10 (fp16) of a score of magnitude 4 where the fp32 sum order moves a
+    rounding, and one rounding of p and of the result, 2e-2 in all."""
+    import torch
+    tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dt]
+    N = B * H * T
+    # q, k and v share one allocation with a NaN before k and after each: what
+    # is read past a tensor's end must not reach the result
+    g = torch.Generator().manual_seed(hd * 1000 + T)
+    x = [torch.randn(N * hd, generator=g).to(tdt) for _ in range(3)]
+    pad = 16
+    buf = torch.full((3 * (N * hd + 2 * pad),), float("nan"), dtype=tdt)
+    off = [i * ((N * hd + 2 * pad) // 16 * 16) for i in range(3)]
+    for o, t in zip(off, x):
+        buf[o:o + N * hd] = t
+    dev = buf.cuda()
+    q, k, v = (dev[o:o + N * hd] for o in off)
+    ctx = empty((B * T, H * hd), dt)
+    (hip.attention_textbook if textbook else hip.attention)(q, k, v, ctx, B, H, T, hd, causal)
+    qd, kd, vd = (t.double().view(B * H, T, hd) for t in x)
+    keys = kd.transpose(1, 2) if textbook else x[1].double().view(hd, B * H, T).permute(1, 0, 2)
+    scale = float(torch.tensor(1 / np.sqrt(hd), dtype=torch.float32).to(tdt))
+    s = ((qd @ keys.contiguous()).to(tdt).double() * scale).to(tdt).double()
+    if causal:
+        s = s.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -float("inf"))
+    ref = (torch.softmax(s, -1) @ vd).view(B, H, T, hd).permute(0, 2, 1, 3).reshape(B * T, H * hd)
+    err = float((ctx.cpu().double() - ref).abs().max() / ref.abs().max())
+    assert err <= (2e-5 if dt == F32 else 2e-2), err
 
 
 @pytest.mark.parametrize("dt", [F16, BF16])
