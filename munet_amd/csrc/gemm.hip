@@ -278,11 +278,16 @@ hipError_t launch_cfg(const void *A, const void *Bt, int M, int N, int K, long l
   else vec = vec && (lda % E == 0) && (sa % E == 0);
   dim3 grid(tiles, 1, batch);
   const ConvArgs none{};
-  // Instantiated variants: the aligned (VEC) path for every tile; the
+  // Instantiated variants, 16-bit: the aligned (VEC) path for every tile; the
   // unaligned path only for the 64x64 tile (host falls back to it); the conv
   // loader for tiles up to 256x128.
   constexpr bool kSmall = (BM == 64 && BN == 64);
-  if (cv) {
+  if constexpr (DT == F32) {
+    // whole 16-byte chunks run on gemm_f32.hip
+    if constexpr (!kSmall) return hipErrorInvalidValue;
+    else if (cv) launch_one<DT, BM, BN, WGM, WGN, false, true>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, *cv);
+    else launch_one<DT, BM, BN, WGM, WGN, false, false>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, none);
+  } else if (cv) {
     if constexpr (BM * BN <= 256 * 128 && WGM * WGN == 4) {
       if (vec) launch_one<DT, BM, BN, WGM, WGN, true, true>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, *cv);
       else if constexpr (kSmall) launch_one<DT, BM, BN, WGM, WGN, false, true>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, *cv);
@@ -327,14 +332,22 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   bool vec = (ldb % E == 0) && (sb % E == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)Bt % 16 == 0);
   if (cv) vec = vec && (cv->iC % E == 0) && (cv->ldx % E == 0);
   else vec = vec && (lda % E == 0) && (sa % E == 0);
-  if (!vec) best = 4;
-  if ((cv || DT == F32) && best == 0) best = 1;  // 256x256 only for 16-bit plain GEMMs
-  if ((cv || DT == F32) && best >= 5) best = 2;  // 8-wave tiles only for 16-bit plain GEMMs
+  if (!vec || DT == F32) best = 4;
+  if (cv && best == 0) best = 1;  // 256x256 only for plain GEMMs
+  if (cv && best >= 5) best = 2;  // 8-wave tiles only for plain GEMMs
   switch (best) {
-  case 0: return launch_cfg<DT, 256, 256, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-  case 1: return launch_cfg<DT, 256, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-  case 2: return launch_cfg<DT, 128, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-  case 3: return launch_cfg<DT, 128, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+  case 0:
+    if constexpr (DT != F32) return launch_cfg<DT, 256, 256, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    return hipErrorInvalidValue;
+  case 1:
+    if constexpr (DT != F32) return launch_cfg<DT, 256, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    return hipErrorInvalidValue;
+  case 2:
+    if constexpr (DT != F32) return launch_cfg<DT, 128, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    return hipErrorInvalidValue;
+  case 3:
+    if constexpr (DT != F32) return launch_cfg<DT, 128, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    return hipErrorInvalidValue;
   case 5:
     if constexpr (DT != F32) return launch_cfg<DT, 256, 128, 4, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
     return hipErrorInvalidValue;
@@ -356,17 +369,17 @@ hipError_t gemm_nt(int dt, const void *A, const void *Bt, int M, int N, int K, l
   if (tile_hint < 0) {
     // MUNET_HIP_GEMM_TILE forces a kernel and block tile for tests and tuning:
     // 0-6 direct-to-LDS kernel, 100-107 general kernel, 200-203, 207-212,
-    // 216, 217 and 219 pipelined kernel.  Read at every call so a process can
+    // 216, 217 and 219 pipelined kernel, 300-302 fp32 kernel.  Read at every call so a process can
     // switch it between calls; any other code is an error.
     const char *force = std::getenv("MUNET_HIP_GEMM_TILE");
     if (force && *force) {
       tile_hint = std::atoi(force);
-      const bool known = (tile_hint >= 0 && tile_hint <= 6) || (tile_hint >= 100 && tile_hint <= 107) ||
+      const bool known = (tile_hint >= 0 && tile_hint <= 6) || (tile_hint >= 300 && tile_hint <= 302) || (tile_hint >= 100 && tile_hint <= 107) ||
                          (tile_hint >= 200 && tile_hint <= 203) || (tile_hint >= 207 && tile_hint <= 212) ||
                          tile_hint == 216 || tile_hint == 217 || tile_hint == 219;
       if (!known)
         throw std::invalid_argument(std::string("MUNET_HIP_GEMM_TILE=") + force +
-                                    " names no GEMM tile (0-6, 100-107, 200-203, 207-212, 216, 217, 219)");
+                                    " names no GEMM tile (0-6, 100-107, 200-203, 207-212, 216, 217, 219, 300-302)");
     }
   }
   // <0: the pipelined 16-bit kernel when the operands allow it, else the
@@ -377,6 +390,11 @@ hipError_t gemm_nt(int dt, const void *A, const void *Bt, int M, int N, int K, l
   // small fp32 products: one workgroup per 16x16 tile, K split over its waves
   if (tile_hint < 0 && gemm_skinny_ok(dt, A, Bt, M, N, K, lda, ldb, batch, ep))
     return gemm_skinny(A, Bt, M, N, K, lda, ldb, ep, st);
+  if (dt == F32 && (tile_hint < 0 || tile_hint >= 300) && gemm_f32_ok(A, Bt, K, lda, ldb, sa, sb, nullptr) &&
+      !ep.stats_out && !ep.ln_stats)
+    return gemm_f32((const float *)A, (const float *)Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, nullptr,
+                    tile_hint - 300, st);
+  if (tile_hint >= 300) tile_hint = -1;
   const bool pipe = gemm_pipe_ok(dt, A, Bt, M, N, K, lda, ldb, sa, sb);
   const bool fold = ep.stats_out || ep.ln_stats;
   if (pipe && (tile_hint < 0 || tile_hint >= 200 || fold))
@@ -450,7 +468,10 @@ hipError_t gemm_splitk(int dt, const void *A, const void *Bt, int M, int N, int 
   EpiArgs part;  // raw fp32 partial products, slice s at ws + s M N
   part.out = ws;
   part.ldc = N;
-  hipError_t e = launch_dt<F32>(A, Bt, M, N, Kc, K, K, S, Kc, Kc, long(M) * N, part, nullptr, -1, st);
+  const hipError_t e =
+      gemm_f32_ok(A, Bt, Kc, K, K, Kc, Kc, nullptr)
+          ? gemm_f32((const float *)A, (const float *)Bt, M, N, Kc, K, K, S, Kc, Kc, long(M) * N, part, nullptr, -1, st)
+          : launch_dt<F32>(A, Bt, M, N, Kc, K, K, S, Kc, Kc, long(M) * N, part, nullptr, -1, st);
   if (e != hipSuccess) return e;
   const long items = long(M) * ((N + 3) / 4);
   hipLaunchKernelGGL(splitk_reduce_kernel<F32>, dim3(unsigned((items + 3) / 4)), dim3(256), 0, st, ws, S, M, N, ep);
@@ -535,7 +556,10 @@ hipError_t conv_nhwc(int dt, const void *x, const void *w_ohwi, const ConvArgs &
   if (tile_hint < 0 && !general && gemm_pipe_conv_ok(dt, x, w_ohwi, cv))
     return gemm_pipe_conv(dt, x, w_ohwi, cv, oC, ep, st);
   switch (dt) {
-  case F32: return launch_dt<F32>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);
+  case F32:
+    if (tile_hint < 0 && gemm_f32_ok(x, w_ohwi, K, 0, K, 0, 0, &cv))
+      return gemm_f32((const float *)x, (const float *)w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, -1, st);
+    return launch_dt<F32>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);
   case F16: return launch_dt<F16>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);
   case BF16: return launch_dt<BF16>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);
   default: return hipErrorInvalidValue;

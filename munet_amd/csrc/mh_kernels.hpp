@@ -143,6 +143,11 @@ hipError_t gemm_skinny(const void *A, const void *Bt, int M, int N, int K, long 
                        hipStream_t st);
 hipError_t conv_nhwc(int dt, const void *x, const void *w_ohwi, const ConvArgs &cv, int oC, const EpiArgs &ep,
                      int tile_hint, hipStream_t st);
+// fp32 GEMM / NHWC convolution (cv) on whole 16-byte chunks (gemm_f32.hip);
+// tile: < 0 automatic, 0 64x64, 1 32x64, 2 32x32.
+bool gemm_f32_ok(const void *A, const void *Bt, int K, long lda, long ldb, long sa, long sb, const ConvArgs *cv);
+hipError_t gemm_f32(const float *A, const float *Bt, int M, int N, int K, long lda, long ldb, int batch, long sa,
+                    long sb, long sc, const EpiArgs &ep, const ConvArgs *cv, int tile, hipStream_t st);
 // Split-K for small fp32 products (gemm.hip): the slice count for M x N x K
 // (1: no split), and the product itself through an fp32 workspace of
 // S * M * N floats (row-major epilogue only).

@@ -8,6 +8,7 @@ kernel there)."""
 import pytest
 
 from munet_amd import synth
+from munet_amd.backend import empty
 from util import assert_close, rand
 
 pytestmark = pytest.mark.gpu
@@ -131,3 +132,42 @@ def test_f16_fixed_programs_bit_identical_to_general(tile, hip, monkeypatch):
             torch.cuda.synchronize()
             outs.append(out.view(torch.int16).clone())
         assert torch.equal(outs[0], outs[1]), f"tile {tile} act={act} resid={resid is not None} bias={use_bias}"
+
+
+@pytest.mark.parametrize("tile", [None, 300, 301, 302])
+@pytest.mark.parametrize("M,K,N", [(65, 32, 64), (64, 36, 68), (31, 4, 33), (130, 100, 200), (1, 64, 5), (300, 516, 31)])
+@pytest.mark.parametrize("batched", [False, True])
+def test_f32_tiles(hip, monkeypatch, tile, M, K, N, batched):
+    """The fp32 kernel's tiles at their edges: one slab, an odd and an even
+    number of 32-wide slabs, K tails of 4 values, ragged rows and columns, batch
+    slices.  Against float64; a sum of K products rounds at most K times, each
+    by 2^-24 of a partial sum, and M N outputs of standard normal operands stay
+    below 6 sqrt(K): bound 6 sqrt(K) K 2^-24."""
+    import torch
+    if tile is not None:
+        monkeypatch.setenv("MUNET_HIP_GEMM_TILE", str(tile))
+    nb = 3 if batched else 1
+    g = torch.Generator().manual_seed(M * 7 + K)
+    a, b = torch.randn(nb, M, K, generator=g), torch.randn(nb, N, K, generator=g)
+    out = empty((nb, M, N), synth.F32)
+    hip.batched_matmul(a.cuda(), b.cuda(), out, nb, M, K, N, False, True, M * K, N * K, M * N)
+    ref = a.double() @ b.double().transpose(1, 2)
+    assert float((out.cpu().double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("B,iC,H,W,oC,k,s,p", [(2, 4, 9, 7, 33, 3, 1, 1), (1, 12, 8, 8, 64, 5, 2, 2), (3, 36, 5, 6, 20, 3, 2, 1),
+                                               (1, 64, 16, 16, 128, 3, 1, 1), (2, 32, 4, 4, 8, 1, 1, 0), (1, 8, 7, 7, 8, 7, 1, 3)])
+def test_f32_conv_columns(hip, B, iC, H, W, oC, k, s, p):
+    """The fp32 implicit-GEMM convolution's stepped (tap, channel) columns:
+    channel counts below, at and above a 32-wide slab that divide it or not,
+    1x1 to 7x7 taps, strides, padding.  Against float64, bound as in
+    test_f32_tiles with K = k k iC."""
+    import torch
+    g = torch.Generator().manual_seed(iC * 10 + k)
+    x, w, b = torch.randn(B, iC, H, W, generator=g), torch.randn(oC, iC, k, k, generator=g), torch.randn(oC, generator=g)
+    ref = torch.nn.functional.conv2d(x.double(), w.double(), b.double(), stride=s, padding=p).permute(0, 2, 3, 1)
+    out = empty(tuple(ref.shape), synth.F32)
+    hip.conv2d_nhwc(x.permute(0, 2, 3, 1).contiguous().cuda(), w.permute(0, 2, 3, 1).contiguous().cuda(), b.cuda(), out, B,
+                    iC, H, W, oC, k, k, s, p)
+    K = iC * k * k
+    assert float((out.cpu().double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24 + 1e-6
