@@ -16,9 +16,11 @@ int pipe_wave_cols(int tile) {
   switch (tile) {
   case 0: case 7: case 9: return 64;
   case 3: case 8: case 10: case 11: case 17: return 48;
+  case 21: case 22: case 24: return 48;
+  case 26: return 16;
   case 16: return 96;
   case 19: return 144;
-  default: return 32;  // 1 (128x64), 2 (64x64), 12 (128x64)
+  default: return 32;  // 1 (128x64), 2 (64x64), 12 (128x64), 20 (64x64), 23 (32x64), 25 (128x64)
   }
 }
 
@@ -54,9 +56,31 @@ int auto_tile(bool dma, int M, int N, int K, int batch) {
   return (t128 >= 640 || (K >= 2048 && t128 >= 128)) ? 0 : (t64 >= 256 ? 1 : 2);
 }
 
+// Small tiles with many stages (gemm_pipe_deep.hip) while they give at most
+// one workgroup per CU, the smallest first: below that count a smaller tile
+// spreads the same steps over more CUs (237 x 768 x 3072: 32x32 10.0 us, 32x64
+// 11.3, 64x64 13.0, 64x96 15.4), above it the workgroups take turns (512 x
+// 768 x 3072: 32x32 17.7, 32x64 11.5).  -1: none fits, the block tiles.
+// A tile's wave tiles must cover whole groups of the LayerNorm partials.
+int deep_tile(int kind, int M, int N, int batch, const EpiArgs &ep) {
+  if (kind == PK_BIAS_NT || ep.mode == EPI_CONVT) return -1;
+  const bool ln = ep.ln_stats != nullptr, st = ep.stats_out != nullptr;
+  struct T { int tile, bm, bn; };
+  const T order[7] = {{26, 32, 32}, {24, 32, 48}, {23, 32, 64}, {21, 64, 48}, {20, 64, 64}, {22, 64, 96}, {25, 128, 64}};
+  for (const T &t : order) {
+    if (long((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch > 256) continue;
+    if (ln && (t.tile == 26 || t.tile == 23)) continue;
+    if (t.bn == 48 && !st) continue;
+    if (t.tile == 22 && N % 96) continue;
+    if (st && pipe_wave_cols(t.tile) % ep.stats_cols) continue;
+    return t.tile;
+  }
+  return -1;
+}
+
 // The tiles with fixed epilogue programs (gemm_pipe_fixed_*.hip).
 bool fixed_tile(int tile) {
-  return (tile >= 0 && tile <= 3) || tile == 8 || tile == 9 || tile == 16 || tile == 17 || tile == 19;
+  return (tile >= 0 && tile <= 3) || tile == 8 || tile == 9 || tile == 16 || tile == 17 || tile == 19 || tile >= 20;
 }
 
 // The epilogue program for these arguments: a fixed program for the
@@ -98,6 +122,7 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // 11.5 -> 10.4, up0 19.1 -> 15.1 against 128x64; the direct-to-LDS 128x128
   // 20-31 us)
   if (tile < 0 && ep.mode == EPI_CONVT) tile = 2;
+  if (tile < 0 && dma) tile = deep_tile(kind, M, N, batch, ep);
   if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = auto_tile(dma, M, N, K, batch);
   if (tile >= 7 && !dma) tile = 0;
   if (tile == 19 && (M % 128 || N % 288)) tile = auto_tile(dma, M, N, K, batch);
@@ -105,6 +130,11 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // groups: move to the nearest tile whose wave-tile width is a multiple
   if (ep.stats_out && pipe_wave_cols(tile) % ep.stats_cols)
     tile = ep.stats_cols == 48 ? (dma ? 8 : 3) : ep.stats_cols == 64 ? (dma ? 9 : 0) : 2;
+  if (tile >= 20) {
+    // a forced tile that has not this program takes 64x64
+    const bool ln = ep.ln_stats != nullptr, no = (ln && (tile == 23 || tile == 26)) || (!ep.stats_out && (tile == 21 || tile == 24));
+    return gemm_pipe_deep(DT, kind, no ? 20 : tile, A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st);
+  }
   if (tile == 16 || tile == 17 || tile == 19)
     return gemm_pipe_wide(DT, kind, tile, A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st);
   if (kind > PK_GENERAL && fixed_tile(tile))

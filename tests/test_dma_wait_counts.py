@@ -39,7 +39,7 @@ def _template_args(name):
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-@pytest.mark.parametrize("src", ["gemm_pipe_wide.hip", "gemm_pipe_fixed_dma.hip", "gemm_pipe_conv.hip"])
+@pytest.mark.parametrize("src", ["gemm_pipe_wide.hip", "gemm_pipe_fixed_dma.hip", "gemm_pipe_conv.hip", "gemm_pipe_deep.hip"])
 def test_first_slab_wait_covers_slab0(src, tmp_path):
     s = _asm(src, tmp_path)
     checked = 0
@@ -50,7 +50,11 @@ def test_first_slab_wait_covers_slab0(src, tmp_path):
         ins = [ln.strip() for ln in body.splitlines()
                if ln.strip() and not ln.strip().startswith((";", ".")) and not re.match(r"^\S+:$", ln.strip())]
         first_mfma = next(i for i, x in enumerate(ins) if "mfma" in x)
-        pro = ins[:first_mfma]
+        # (a 32x32 tile's first step issues its loads ahead of its one MFMA per
+        # half: the prologue ends at the barrier that publishes slab 0)
+        first_dma = next(i for i, x in enumerate(ins) if x.startswith("global_load_lds_dwordx4"))
+        barrier = next(i for i, x in enumerate(ins) if i > first_dma and x.startswith("s_barrier"))
+        pro = ins[:min(first_mfma, barrier)]
         # the slabs' 16-byte DMAs (the 4-byte loads issued before them touch
         # the next GEMM's weights; being older, they only add to the wait)
         # (convolutions: the A blocks through the buffer form, padding taps

@@ -171,3 +171,35 @@ def test_f32_conv_columns(hip, B, iC, H, W, oC, k, s, p):
                     iC, H, W, oC, k, k, s, p)
     K = iC * k * k
     assert float((out.cpu().double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24 + 1e-6
+
+
+@pytest.mark.parametrize("tile", list(range(220, 227)))
+def test_deep_tiles(tile, hip, orc, monkeypatch):
+    """The small many-stage tiles (up to 16 stages: products of fewer slabs
+    than stages re-load the last one) at the edges of test_forced_tile's shapes
+    against the oracle, and bit for bit against the 128x128 kernel."""
+    test_forced_tile(tile, hip, orc, monkeypatch)
+    test_tiles_bit_identical_to_128(tile, hip, monkeypatch)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (33, 96, 128), (256, 1024, 64), (257, 1024, 64), (500, 2048, 192), (512, 768, 256),
+                                   (2048, 768, 64), (2049, 768, 64), (300, 4096, 64)])
+def test_deep_tile_choice_bits(M, N, K, hip, monkeypatch):
+    """Both sides of each border of the small-tile choice (at most one tile per
+    CU) give the 128x128 kernel's bits, bias + GELU and bias + residual."""
+    from munet_amd.backend import to_device, to_host
+    for dt in (synth.BF16, synth.F16):
+        x, w, b, r = (to_device(rand(s, dt, i, c), dt) for i, (s, c) in
+                      enumerate([((M, K), 1.0), ((N, K), 0.2), ((N,), 1.0), ((M, N), 1.0)]))
+        for act, resid in ((2, None), (0, r)):
+            outs = []
+            for t in (None, 200):
+                if t is None:
+                    monkeypatch.delenv("MUNET_HIP_GEMM_TILE", raising=False)
+                else:
+                    monkeypatch.setenv("MUNET_HIP_GEMM_TILE", str(t))
+                out = empty((M, N), dt)
+                hip.linear(x, w, b, out, M, K, N, act, resid)
+                hip.synchronize()
+                outs.append(to_host(out, dt))
+            assert (outs[0] == outs[1]).all()
