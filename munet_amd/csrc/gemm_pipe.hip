@@ -37,12 +37,25 @@ int pipe_wave_cols(int tile) {
 //    attention out-projection): direct-to-LDS 128x96, 4 stages, eight waves
 //    (one workgroup per CU, so deep stages and two waves per SIMD hide the
 //    memory latency; out-projection 13.9 -> 12.9 us against four waves);
-//  * otherwise register-staged: 128x128 when N tiles evenly by 128 and there
-//    are >= 2.5 tiles per CU (FFN up, LM head), 128x96 when N tiles evenly by
-//    96 (QKV), else 128x128 / 128x64 / 64x64 by tile count.
+//  * up to 256 128x128 tiles: register-staged 128x128 (1500 x 2304 x 768 13.0
+//    us; 128x96 15.8, direct-to-LDS 128x128 14.0), with a GELU 128x64 (fp16:
+//    64x64), whose two to four workgroups per CU overlap one's epilogue with
+//    another's loop (2048 x 2048 x 512: bf16 12.1 -> 11.3 us, fp16, whose
+//    half-away roundings take more, 25.1 -> 16.3, 128x64 18.3);
+//  * N tiling by 96 into at most two 128x96 tiles per CU: register-staged
+//    128x96 (8192 x 768 x 3072 49.8 us; direct-to-LDS 128x128 55);
+//  * else the direct-to-LDS tile with the least rounds times round time: two
+//    128x128 (two stages) per CU, 256x192 and (whole tiles only) 128x288 one
+//    per CU, a round of 256x192 taking 1.25 to 1.39 and of 128x288 1.15 to 1.25
+//    of a 128x128 round, a last round of at most one 128x128 per CU 0.75 (2000 x 4096 x 1024:
+//    128x128 21.7 us, 256x192 26.8, register-staged 128x64 29.9; 2048 x 5000 x
+//    512: 22.6, 18.7, 22.0; 8192 x 2304 x 768: 50.6, 48.4, 128x288 43.6);
+//  * K % 64 != 0, register-staged: 128x128 when N tiles evenly by 128 and there
+//    are >= 2.5 tiles per CU, 128x96 when N tiles evenly by 96, else 128x128 /
+//    128x64 / 64x64 by tile count.
 // (The vocabulary head, a non-temporal output, takes direct-to-LDS 128x128
 // with two stages: see launch_dt.)
-int auto_tile(bool dma, int M, int N, int K, int batch) {
+int auto_tile(bool dma, int dt, int act, int M, int N, int K, int batch) {
   const long t128 = long((M + 127) / 128) * ((N + 127) / 128) * batch;
   const long t96 = long((M + 127) / 128) * ((N + 95) / 96) * batch;
   const long t64 = long((M + 127) / 128) * ((N + 63) / 64) * batch;
@@ -51,6 +64,16 @@ int auto_tile(bool dma, int M, int N, int K, int batch) {
   const long t288 = long(M / 128) * (N / 288) * batch;
   if (dma && M % 128 == 0 && N % 288 == 0 && t288 >= 232 && t288 <= 256) return 19;
   if (dma && N % 96 == 0 && t96 <= 256) return 17;
+  if (dma && t128 > 128) {
+    if (t128 <= 256) return act != ACT_GELU ? 0 : dt == F16 ? 2 : 1;
+    if (N % 96 == 0 && t96 <= 512) return 3;
+    const long rem = t128 % 512;
+    const double c9 = double(t128 / 512) + (rem > 256 ? 1.0 : rem > 0 ? 0.75 : 0.0);
+    const long n16 = long((M + 255) / 256) * ((N + 191) / 192) * batch;
+    const double c16 = 1.33 * double((n16 + 255) / 256);
+    const double c19 = M % 128 == 0 && N % 288 == 0 ? 1.15 * double((t288 + 255) / 256) : 1e30;
+    return c9 <= c16 && c9 <= c19 ? 9 : c16 <= c19 ? 16 : 19;
+  }
   if (N % 128 == 0 && t128 >= 640) return 0;
   if (N % 96 == 0) return 3;
   return (t128 >= 640 || (K >= 2048 && t128 >= 128)) ? 0 : (t64 >= 256 ? 1 : 2);
@@ -123,9 +146,9 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // 20-31 us)
   if (tile < 0 && ep.mode == EPI_CONVT) tile = 2;
   if (tile < 0 && dma) tile = deep_tile(kind, M, N, batch, ep);
-  if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = auto_tile(dma, M, N, K, batch);
+  if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = auto_tile(dma, DT, ep.act, M, N, K, batch);
   if (tile >= 7 && !dma) tile = 0;
-  if (tile == 19 && (M % 128 || N % 288)) tile = auto_tile(dma, M, N, K, batch);
+  if (tile == 19 && (M % 128 || N % 288)) tile = auto_tile(dma, DT, ep.act, M, N, K, batch);
   // LayerNorm partials of stats_cols columns need wave tiles that cover whole
   // groups: move to the nearest tile whose wave-tile width is a multiple
   if (ep.stats_out && pipe_wave_cols(tile) % ep.stats_cols)

@@ -106,16 +106,18 @@ template <> struct PipeMfma<F16> {
 template <int BM, int BN>
 __device__ __forceinline__ void pipe_tile(int M, int N, int gn, int &m0, int &n0) {
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, ntiles = tiles_m * tiles_n;
-  int pid = blockIdx.x;
   constexpr int GROUP = 8;
-  if (gn > 0 && (ntiles & 7) == 0) {
-    const int t = (pid & 7) * (ntiles >> 3) + (pid >> 3), span = gn * tiles_m;
-    const int g = t / span, r = t - g * span, w = min(gn, tiles_n - g * gn);
+  // XCD x walks the tiles from x q + min(x, r) on (q or, for the first r XCDs,
+  // q + 1 of them)
+  const int xcd = blockIdx.x & 7, q = ntiles >> 3, r8 = ntiles & 7;
+  const int pid = xcd * q + min(xcd, r8) + int(blockIdx.x >> 3);
+  if (gn > 0) {
+    const int span = gn * tiles_m;
+    const int g = pid / span, r = pid - g * span, w = min(gn, tiles_n - g * gn);
     m0 = (r / w) * BM;
     n0 = (g * gn + r % w) * BN;
     return;
   }
-  if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
   const int span = GROUP * tiles_n, gid = pid / span, fm = gid * GROUP, gs = min(tiles_m - fm, GROUP);
   m0 = (fm + (pid % span) % gs) * BM;
   n0 = ((pid % span) / gs) * BN;
