@@ -1758,8 +1758,7 @@ struct mh_decoder {
     if (logits_out)
       hip_check(hipMemcpyAsync(logits_out, out, size_t(B) * T0 * V * es, hipMemcpyDeviceToHost, e.stream), "logits D2H");
     // the next input: each sequence's greedy choice at its last position
-    for (int b = 0; b < B; ++b)
-      hip_check(mh::argmax_rows(dt, out + (size_t(b) * T0 + T0 - 1) * V * es, ids + b, 1, V, e.stream), "prefill argmax");
+    hip_check(mh::argmax_rows(dt, out + size_t(T0 - 1) * V * es, ids, B, V, e.stream, long(T0) * V), "prefill argmax");
     const int st[3] = {T0, 0, 0};
     hip_check(hipMemcpyAsync(state, st, sizeof(st), hipMemcpyHostToDevice, e.stream), "decoder state");
     hip_check(hipStreamSynchronize(e.stream), "prefill");

@@ -219,7 +219,8 @@ hipError_t check_f16_rounding(unsigned long long *mismatches, hipStream_t st);
 // stats_cols = D).
 hipError_t embedding(int dt, const int32_t *ids, const void *w, const void *pos, void *out, int n, int V, int D,
                      int T, int *err, hipStream_t st, float *stats = nullptr);
-hipError_t argmax_rows(int dt, const void *x, int32_t *out, int rows, int cols, hipStream_t st);
+// rows ld values apart (0: cols)
+hipError_t argmax_rows(int dt, const void *x, int32_t *out, int rows, int cols, hipStream_t st, long ld = 0);
 // Measured matrix-core peak (peak.hip): FLOP/s of a full grid of independent
 // 16x16x32 MFMAs (bf16 or fp16), `iters` loop trips per wave.
 hipError_t mfma_peak(int dt, int iters, double *flops_per_s, hipStream_t st);

@@ -364,6 +364,30 @@ def test_argmax(hip, dt):
 
 
 @pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("cols", [1, 8, 63, 1000, 1024, 1025, 4104, 32000, 40007])
+def test_argmax_rows(hip, dt, cols):
+    """Both row widths and both load widths: ties far apart give the first
+    index, NaN never wins, rows of -inf and of NaN give index 0, whole numbers
+    exactly."""
+    x = rand((6, cols), dt, 94)
+    f = dec(x, dt)
+    f[1, cols // 3] = f[1, cols - 1] = 60.0
+    f[2, 0] = f[2, cols // 2] = f[2, cols - 1] = 60.0
+    f[3, :] = -np.inf
+    x = synth.encode(f, dt)
+    nan = {F32: np.float32(np.nan), F16: np.uint16(0x7e00), BF16: np.uint16(0x7fc0)}[dt]
+    x[4, :] = nan
+    x[5, ::2] = nan
+    ref = np.argmax(f, axis=1)
+    ref[4] = 0
+    odd = np.where(np.arange(cols) % 2 == 1, f[5], -np.inf)
+    ref[5] = int(np.argmax(odd)) if cols > 1 else 0
+    out = empty((6,), I32)
+    hip.argmax(to_device(x, dt), out, 6, cols)
+    assert np.array_equal(to_host(out, I32), ref)
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("B,iC,H,W,oC,k,s,p", [(2, 3, 9, 9, 4, 3, 1, 1), (2, 3, 9, 9, 4, 3, 2, 1),
                                                (1, 16, 12, 10, 32, 3, 1, 1), (2, 8, 8, 8, 16, 1, 1, 0),
                                                (1, 32, 16, 16, 16, 3, 2, 1),
