@@ -192,23 +192,134 @@ layernorm_long_kernel(const typename Store<DT>::T *__restrict__ x, const typenam
   for (int c = lane; c < cols; c += 64) yr[c] = S::enc((S::dec(xr[c]) - mean) * inv * S::dec(w[c]) + S::dec(b[c]));
 }
 
-template <int DT>
-__global__ void __launch_bounds__(256)
-softmax_kernel(const typename Store<DT>::T *__restrict__ x, typename Store<DT>::T *__restrict__ y, int rows, int cols) {
+// One row per TH threads (256-thread workgroups of four rows for TH = 64),
+// the row in registers: NV groups of E consecutive values per thread, group
+// (k TH + t) E, all loaded before the first reduction.  The exponentials are
+// doubles, as the reference's, and are taken once: kept as doubles between the
+// sum and the division.  Bound: HBM (one read, one write).  The kernel this
+// replaces ran one wave per row in three passes over memory with both
+// exponentials recomputed (1000 rows of 5000 floats 84 us, one wave per SIMD).
+template <int DT, int TH, int NV, int E>
+__global__ void __launch_bounds__(TH < 256 ? 256 : TH)
+softmax_row_kernel(const typename Store<DT>::T *__restrict__ x, typename Store<DT>::T *__restrict__ y, int rows, int cols) {
   typedef Store<DT> S;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
+  constexpr int NW = TH / 64;
+  __shared__ float smx[NW];
+  __shared__ double ssum[NW];
+  const int tid = TH == 64 ? threadIdx.x & 63 : threadIdx.x;
+  const int row = TH == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  if (row >= rows) return;  // TH = 64: whole waves, which share nothing
   const typename Store<DT>::T *xr = x + long(row) * cols;
+  float v[NV][E];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int c = (k * TH + tid) * E;
+    if (c < cols) {
+      if constexpr (E == 4) ld4<DT>(xr + c, v[k]);
+      else v[k][0] = S::dec(xr[c]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[k][e] = -INFINITY;
+    }
+  }
   float mx = -INFINITY;
-  for (int c = lane; c < cols; c += 64) mx = fmaxf(mx, S::dec(xr[c]));
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+#pragma unroll
+    for (int e = 0; e < E; ++e) mx = fmaxf(mx, v[k][e]);
   mx = wave_max(mx);
-  double sum = 0.0;
-  for (int c = lane; c < cols; c += 64) sum += exp(double(S::dec(xr[c])) - double(mx));
+  if constexpr (NW > 1) {
+    if ((tid & 63) == 0) smx[tid >> 6] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mx = fmaxf(mx, smx[w]);
+  }
+  double ex[NV][E], sum = 0.0;
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if ((k * TH + tid) * E < cols)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        ex[k][e] = exp(double(v[k][e]) - double(mx));
+        sum += ex[k][e];
+      }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  if constexpr (NW > 1) {
+    if ((tid & 63) == 0) ssum[tid >> 6] = sum;
+    __syncthreads();
+    sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sum += ssum[w];
+  }
   typename Store<DT>::T *yr = y + long(row) * cols;
-  for (int c = lane; c < cols; c += 64) yr[c] = S::enc(float(exp(double(S::dec(xr[c])) - double(mx)) / sum));
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int c = (k * TH + tid) * E;
+    if (c < cols) {
+      float o[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) o[e] = float(ex[k][e] / sum);
+      if constexpr (E == 4) st4<DT>(yr + c, o);
+      else yr[c] = S::enc(o[0]);
+    }
+  }
+}
+
+// Rows past the registers of 1024 threads: three passes of the row, one
+// workgroup of 1024 threads per row.
+template <int DT>
+__global__ void __launch_bounds__(1024)
+softmax_long_kernel(const typename Store<DT>::T *__restrict__ x, typename Store<DT>::T *__restrict__ y, int cols) {
+  typedef Store<DT> S;
+  __shared__ float smx[16];
+  __shared__ double ssum[16];
+  const int tid = threadIdx.x;
+  const typename Store<DT>::T *xr = x + long(blockIdx.x) * cols;
+  float mx = -INFINITY;
+  for (int c = tid; c < cols; c += 1024) mx = fmaxf(mx, S::dec(xr[c]));
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) smx[tid >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) mx = fmaxf(mx, smx[w]);
+  double sum = 0.0;
+  for (int c = tid; c < cols; c += 1024) sum += exp(double(S::dec(xr[c])) - double(mx));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  if ((tid & 63) == 0) ssum[tid >> 6] = sum;
+  __syncthreads();
+  sum = 0.0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) sum += ssum[w];
+  typename Store<DT>::T *yr = y + long(blockIdx.x) * cols;
+  for (int c = tid; c < cols; c += 1024) yr[c] = S::enc(float(exp(double(S::dec(xr[c])) - double(mx)) / sum));
+}
+
+// Threads per row by its length: a wave to 512 values (eight per lane), 256
+// threads to 4096 (sixteen), 1024 to 16384; groups of four values where rows
+// and pointers allow 4-value accesses.
+template <int DT>
+hipError_t softmax_dt(const void *x, void *y, int rows, int cols, hipStream_t st) {
+  typedef typename Store<DT>::T T;
+  const T *X = (const T *)x;
+  T *Y = (T *)y;
+  const bool vec = cols % 4 == 0 && (uintptr_t)x % (4 * sizeof(T)) == 0 && (uintptr_t)y % (4 * sizeof(T)) == 0;
+#define MH_SM(TH, N)                                                                                                  \
+  {                                                                                                                   \
+    const dim3 g(TH == 64 ? (rows + 3) / 4 : rows), b(TH == 64 ? 256 : TH);                                           \
+    if (vec) hipLaunchKernelGGL((softmax_row_kernel<DT, TH, N / 4, 4>), g, b, 0, st, X, Y, rows, cols);               \
+    else hipLaunchKernelGGL((softmax_row_kernel<DT, TH, N, 1>), g, b, 0, st, X, Y, rows, cols);                       \
+  }
+  if (cols <= 256) MH_SM(64, 4)
+  else if (cols <= 512) MH_SM(64, 8)
+  else if (cols <= 2048) MH_SM(256, 8)
+  else if (cols <= 4096) MH_SM(256, 16)
+  else if (cols <= 8192) MH_SM(1024, 8)
+  else if (cols <= 16384) MH_SM(1024, 16)
+  else hipLaunchKernelGGL((softmax_long_kernel<DT>), dim3(rows), dim3(1024), 0, st, X, Y, cols);
+#undef MH_SM
+  return hipGetLastError();
 }
 
 template <int DT>
@@ -263,14 +374,12 @@ hipError_t layernorm(int dt, const void *x, const void *w, const void *b, void *
 
 hipError_t softmax_rows(int dt, const void *x, void *y, int rows, int cols, hipStream_t st) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
-  dim3 grid((rows + 3) / 4), block(256);
   switch (dt) {
-  case F32: hipLaunchKernelGGL(softmax_kernel<F32>, grid, block, 0, st, (const float *)x, (float *)y, rows, cols); break;
-  case F16: hipLaunchKernelGGL(softmax_kernel<F16>, grid, block, 0, st, (const uint16_t *)x, (uint16_t *)y, rows, cols); break;
-  case BF16: hipLaunchKernelGGL(softmax_kernel<BF16>, grid, block, 0, st, (const uint16_t *)x, (uint16_t *)y, rows, cols); break;
+  case F32: return softmax_dt<F32>(x, y, rows, cols, st);
+  case F16: return softmax_dt<F16>(x, y, rows, cols, st);
+  case BF16: return softmax_dt<BF16>(x, y, rows, cols, st);
   default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 }  // namespace mh

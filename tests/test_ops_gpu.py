@@ -243,6 +243,50 @@ def test_softmax(hip, orc, dt, rows, cols):
 
 
 @pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("rows,cols", [(1, 8), (5, 16), (3, 2056), (700, 40), (33, 2048), (9, 4104), (2, 12), (300, 1), (4, 9)])
+def test_row_broadcast_chunks(hip, orc, dt, rows, cols):
+    """[rows, cols] op [cols]: the 16-byte-chunk kernel (rows narrower and
+    wider than a workgroup, row counts that are no multiple of its step) and
+    the scalar one (odd widths, and a row that starts off a 16-byte boundary)
+    against the oracle, bit for bit (one rounding of the same float op)."""
+    a, b = rand((rows, cols), dt, 12), rand((cols,), dt, 13)
+    info = BroadcastInfo(*compute_broadcast((rows, cols), contiguous_strides((rows, cols)), (cols,), [1]))
+    ad, bd = to_device(a, dt), to_device(b, dt)
+    off = to_device(np.concatenate([b[:1], b]), dt)[1:]  # not 16-byte aligned
+    for call, ref in ((hip.add, orc.add(a, b, dt)), (hip.mul, orc.mul(a, b, dt)), (hip.sub, orc.sub(a, b, dt))):
+        for right in (bd, off):
+            out = empty((rows, cols), dt)
+            call(ad, right, out, info)
+            assert np.array_equal(to_host(out, dt), ref)
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("cols", [1, 5, 256, 260, 513, 2049, 4096, 4100, 8193, 16384, 16385, 30001])
+def test_softmax_rows(hip, dt, cols):
+    """Each thread count per row at its edges, aligned and odd lengths, rows
+    that fill no workgroup; -inf entries give exactly zero, a row with NaN,
+    with +inf or of -inf alone is NaN throughout, as exp(x - max) / sum in
+    doubles gives.  Against float64 with one rounding to the dtype (and the
+    float32 before it): 2^-23 / 2^-10 / 2^-8 of each value, plus half a
+    subnormal half ulp 2^-25 in fp16."""
+    import torch
+    x = rand((5, cols), dt, 51, 4.0)
+    f = dec(x, dt)
+    f[1, : cols // 2] = -np.inf
+    f[2, cols // 2] = np.inf
+    f[3, :] = -np.inf
+    x = synth.encode(f, dt)
+    x[4, cols - 1] = {F32: np.float32(np.nan), F16: np.uint16(0x7e00), BF16: np.uint16(0x7fc0)}[dt]
+    out = empty((5, cols), dt)
+    hip.softmax(to_device(x, dt), out, 5, cols)
+    y = dec(to_host(out, dt), dt)
+    ref = torch.softmax(torch.from_numpy(dec(x, dt)), -1).numpy()
+    assert np.isnan(y[2:]).all()
+    tol = {F32: 2.0 ** -23, F16: 2.0 ** -10, BF16: 2.0 ** -8}[dt]
+    assert (np.abs(y[:2] - ref[:2]) <= tol * ref[:2] + (2.0 ** -24 if dt == F16 else 1e-38)).all()
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("op", [ADD, SUB, MUL, DIV])
 @pytest.mark.parametrize("sa,sb", [((4, 5, 6), (4, 5, 6)), ((7, 9), (9,)), ((3, 1, 5), (1, 4, 1)), ((6,), (2, 3, 6))])
 def test_binary_broadcast(hip, orc, dt, op, sa, sb):
