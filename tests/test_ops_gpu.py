@@ -574,6 +574,25 @@ def test_pool_upsample_concat(hip, orc, dt):
     assert np.array_equal(to_host(un, dt).transpose(0, 3, 1, 2), orc.upsample2d(x, 2, dt))
 
 
+@pytest.mark.parametrize("dt", [F32, BF16, I32])
+@pytest.mark.parametrize("batch,rows,cols", [(1, 64, 64), (2, 65, 72), (2, 72, 65), (3, 8, 8), (1, 9, 200), (2, 128, 9), (3, 15, 130),
+                                             (2, 1000, 9), (1, 200, 100), (1, 1, 5), (2, 24, 1000), (1, 1000, 24), (2, 130, 63)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_transpose2d(hip, dt, batch, rows, cols, shift):
+    """Chunked and scalar loads and stores (lengths that are multiples of a
+    16-byte chunk or not, storages that start on a boundary or one value off
+    it), ragged tiles, and the flat path of narrow slices: exact, and nothing
+    written past the output."""
+    x = rand((batch, rows, cols), dt, 131) if dt != I32 else np.arange(batch * rows * cols, dtype=np.int32).reshape(batch, rows, cols)
+    n = x.size
+    src = to_device(np.concatenate([x.reshape(-1)[:1]] * shift + [x.reshape(-1)]), dt)[shift:]
+    guard = to_device(np.zeros(n + shift + 16, x.dtype), dt)
+    out = guard[shift:shift + n]
+    hip.transpose2d(src, out, batch, rows, cols)
+    assert np.array_equal(to_host(out, dt).reshape(batch, cols, rows), x.transpose(0, 2, 1))
+    assert not to_host(guard[shift + n:], dt).any() and not to_host(guard[:shift], dt).any()
+
+
 @pytest.mark.parametrize("dt", DTS + [I32])
 def test_to_contiguous(hip, dt):
     x = rand((4, 5, 6), dt, 130) if dt != I32 else np.arange(120, dtype=np.int32).reshape(4, 5, 6)
