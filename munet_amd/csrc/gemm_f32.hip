@@ -10,24 +10,28 @@
 // fragment, so what decides is that no wave waits between slabs, and how
 // evenly the tiles spread over 256 CUs:
 //   * slabs double-buffered in LDS, the two after next in registers; every
-//     global load is unconditional (clamped addresses) and what lies outside
-//     becomes zero only when the chunk is stored, so nothing waits beside the
-//     load; one barrier per slab, waiting for LDS only, with the second half's
+//     load is unconditional, through buffer resources that return zeros for
+//     what lies outside; one barrier per slab, waiting for LDS only, with the second half's
 //     MFMAs after it while the next slab's fragments are read;
 //   * the four MFMAs of a 16-byte chunk interleaved over all fragments;
 //   * tiles 64x64, 32x64 and 32x32 on four waves, by the work of the busiest
 //     CU (auto_tile).  128x128 and 128x64 tiles, on four or eight waves,
-//     reached the same 120 TFLOP/s on 4096 x 4096 x 1024 and were behind on
-//     every smaller product (fewer, coarser tiles).
+//     were no faster on 4096 x 4096 x 1024 and behind on every smaller product
+//     (fewer, coarser tiles), and four slabs in registers changed nothing.
+// On 4096 x 4096 x 1024 (128 TFLOP/s) the matrix cores were busy 76% of the
+// kernel before the buffer resources replaced 20 VALU instructions per slab
+// (287 -> 269 us).
 // Measured against the 64x64 general kernel that these products ran on
-// (conditional loads, one slab ahead): 2000 x 1536 x 512 42.3 -> 36.5 us, 2000
-// x 512 x 2048 55.8 -> 43, 1000 x 5000 x 768 93 -> 73; the convolution 16 x 56
-// x 56 x 64 -> 128 146 -> 90.
+// (conditional loads, one slab ahead): 2000 x 1536 x 512 42.3 -> 35 us, 2000
+// x 512 x 2048 55.8 -> 40.5, 1000 x 5000 x 768 93 -> 68; the convolution 16 x 56
+// x 56 x 64 -> 128 146 -> 86.
 //
 // Convolution: the A loader gathers im2col chunks (4 channels of one filter
 // tap) from the NHWC activation; a thread stages the same K column of one or
 // two output pixels and steps its (tap, channel) state by 32 channels per slab
 // without dividing.
+#include <algorithm>
+
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
 #include "gemm_common.hpp"
@@ -36,10 +40,6 @@ namespace mh {
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x4 ldg16(const float *p) {
-  return *(const __attribute__((address_space(1))) u32x4 *)(p);
-}
-
 // Barrier between LDS writers and readers that leaves global loads in flight.
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
@@ -78,57 +78,73 @@ gemm_f32_kernel(const float *__restrict__ A, const float *__restrict__ Bt, int M
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WGN, wn = wave % WGN, li = lane & 15, lg = lane >> 4;
 
-  // staging: chunk c of rows r0 + i NT / 8 of A and of Bt; rows past M / N are
-  // clamped (they feed outputs that are not stored)
+  // staging: chunk c of rows r0 + i NT / 8 of A and of Bt, by 32-bit byte
+  // offsets into buffer resources over the tile's rows (rows past M / N are
+  // clamped: they feed outputs that are not stored).  What lies outside (K's
+  // tail, slabs past the end, padding taps) gets an offset past the resource's
+  // end, which the hardware returns as zeros: no select per value, and a slab
+  // adds a scalar.  (Selects beside the load waited for it at once, a memory
+  // latency on every slab; beside the LDS store they took as many VALU
+  // instructions as there are MFMAs.)
+  constexpr uint32_t kOut = 0x80000000u;
   const int r0 = tid >> 3, c = tid & 7;
-  const float *ap[ACH], *bp[BCH];
+  uint32_t ao[ACH], bo[BCH];
   int ih0[ACH], iw0[ACH];
+  long abase, alen;
+  if constexpr (CONV) {
+    const int img = cv.oH * cv.oW, b0 = m0 / img;
+    abase = long(b0) * cv.iH * cv.iW * cv.ldx;
+    alen = long(cv.B) * cv.iH * cv.iW * cv.ldx - (cv.ldx - cv.iC) - abase;
 #pragma unroll
-  for (int i = 0; i < ACH; ++i) {
-    const int m = min(m0 + r0 + i * (NT / 8), M - 1);
-    if constexpr (CONV) {
+    for (int i = 0; i < ACH; ++i) {
+      const int m = min(m0 + r0 + i * (NT / 8), M - 1);
       const int ow = m % cv.oW, t = m / cv.oW, oh = t % cv.oH, b = t / cv.oH;
       ih0[i] = oh * cv.s - cv.p;
       iw0[i] = ow * cv.s - cv.p;
-      ap[i] = A + long(b) * cv.iH * cv.iW * cv.ldx;
-    } else {
-      ap[i] = A + long(m) * lda;
+      // element offset of tap (0, 0) (it may lie before the image)
+      ao[i] = uint32_t(((b - b0) * cv.iH + ih0[i]) * cv.iW + iw0[i]) * uint32_t(cv.ldx);
     }
+  } else {
+    abase = long(m0) * lda;
+    alen = long(min(BM, M - m0) - 1) * lda + K;
+#pragma unroll
+    for (int i = 0; i < ACH; ++i) ao[i] = (uint32_t(min(r0 + i * (NT / 8), M - 1 - m0)) * uint32_t(lda) + c * 4) * 4;
   }
 #pragma unroll
-  for (int i = 0; i < BCH; ++i) bp[i] = Bt + long(min(n0 + r0 + i * (NT / 8), N - 1)) * ldb;
-  int k = c * 4;  // this thread's K column of the slab it loads next
+  for (int i = 0; i < BCH; ++i) bo[i] = (uint32_t(min(r0 + i * (NT / 8), N - 1 - n0)) * uint32_t(ldb) + c * 4) * 4;
+  const __amdgpu_buffer_rsrc_t ares = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A + abase), 0,
+                                                                        int(min(alen * 4, 0x7fffffffL)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(Bt + long(n0) * ldb), 0, int(min((long(min(BN, N - n0) - 1) * ldb + K) * 4, 0x7fffffffL)), 0x00020000);
+  int ks = 0;  // first K column of the slab loaded next
   int ic = 0, kh = 0, kw = 0;
   if constexpr (CONV) {
-    const int tap = k / cv.iC;
-    ic = k - tap * cv.iC;
+    const int tap = c * 4 / cv.iC;
+    ic = c * 4 - tap * cv.iC;
     kh = tap / cv.kW;
     kw = tap - kh * cv.kW;
   }
-  // The loaded chunks stay as they arrive until they are stored: what lies
-  // outside (oka, okb false) becomes zero there.  A select beside the load
-  // would wait for it at once (a memory latency on every slab).
   // Slab s is held in set s % 2, requested two steps before it is stored.
   u32x4 ra[2][ACH], rb[2][BCH];
-  bool oka[2][ACH], okb[2];
   auto gload = [&](auto setc) {
     constexpr int d = decltype(setc)::value;
-    okb[d] = k < K;  // K % 4 == 0: a chunk is inside or past the end
-    const int kk = okb[d] ? k : 0;
+    const bool in = ks + c * 4 < K;  // K % 4 == 0: a chunk is inside or past the end
+    if constexpr (CONV) {
+      const uint32_t toff = uint32_t(kh * cv.iW + kw) * uint32_t(cv.ldx) + ic;
 #pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      oka[d][i] = okb[d];
-      if constexpr (CONV) {
-        const int ih = ih0[i] + kh, iw = iw0[i] + kw;
-        oka[d][i] = okb[d] && unsigned(ih) < unsigned(cv.iH) && unsigned(iw) < unsigned(cv.iW);
-        ra[d][i] = ldg16(ap[i] + (oka[d][i] ? (long(ih) * cv.iW + iw) * cv.ldx + ic : 0));
-      } else {
-        ra[d][i] = ldg16(ap[i] + kk);
+      for (int i = 0; i < ACH; ++i) {
+        const bool ok = in && unsigned(ih0[i] + kh) < unsigned(cv.iH) && unsigned(iw0[i] + kw) < unsigned(cv.iW);
+        ra[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ares, ok ? (ao[i] + toff) * 4 : kOut, 0, 0));
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < ACH; ++i)
+        ra[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ares, in ? ao[i] : kOut, ks * 4, 0));
     }
 #pragma unroll
-    for (int i = 0; i < BCH; ++i) rb[d][i] = ldg16(bp[i] + kk);
-    k += BK;
+    for (int i = 0; i < BCH; ++i)
+      rb[d][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(bres, in ? bo[i] : kOut, ks * 4, 0));
+    ks += BK;
     if constexpr (CONV) {
       ic += cs.dic;
       int carry = cs.dkw;
@@ -149,18 +165,12 @@ gemm_f32_kernel(const float *__restrict__ A, const float *__restrict__ Bt, int M
 #pragma unroll
     for (int i = 0; i < ACH; ++i) {
       const int r = r0 + i * (NT / 8);
-      u32x4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = oka[d][i] ? ra[d][i][e] : 0u;
-      buf[r * 8 + (c ^ (r & 7))] = v;
+      buf[r * 8 + (c ^ (r & 7))] = ra[d][i];
     }
 #pragma unroll
     for (int i = 0; i < BCH; ++i) {
       const int r = r0 + i * (NT / 8);
-      u32x4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = okb[d] ? rb[d][i][e] : 0u;
-      buf[BM * 8 + r * 8 + (c ^ (r & 7))] = v;
+      buf[BM * 8 + r * 8 + (c ^ (r & 7))] = rb[d][i];
     }
   };
 
@@ -278,13 +288,14 @@ struct Tile {
   int bm, bn;
   double per;  // time per unit of tile area against 64x64 (a smaller tile reads more operands per output)
 };
-const Tile kTiles[3] = {{64, 64, 1.0}, {32, 64, 1.15}, {32, 32, 1.3}};
+const Tile kTiles[3] = {{64, 64, 1.0}, {32, 64, 1.07}, {32, 32, 1.12}};
 
 // The tile whose busiest CU has the least to do: whole tiles per CU times the
 // tile's area (a CU runs its resident tiles side by side on the same matrix
-// cores).  Both sides at its borders: 2048 x 768 x 3072 is 1.5 64x64 tiles per
-// CU, 108 us, or three 32x64, 97 us; 2000 x 512 x 512 256 64x64 tiles, 14.8
-// us, or 504 32x64, 16.0; 300 x 512 x 512 40 / 80 / 160 tiles, 13.1 / 9.1 / 7.6.
+// cores).  Both sides: 4096 x 4096 x 1024 in 64x64 tiles 269 us, 32x64 288,
+// 32x32 302 (the weights of kTiles); 2048 x 768 x 3072 is 1.5 64x64 tiles per
+// CU, 106 us, or three 32x64, 85; 300 x 512 x 512 40 / 80 / 160 tiles, 12.9 /
+// 8.6 / 8.1.
 int auto_tile(int M, int N, int batch) {
   int best = 0;
   double best_t = 1e30;
@@ -303,7 +314,13 @@ int auto_tile(int M, int N, int batch) {
 
 bool gemm_f32_ok(const void *A, const void *Bt, int K, long lda, long ldb, long sa, long sb, const ConvArgs *cv) {
   const bool b = K > 0 && K % 4 == 0 && ldb % 4 == 0 && sb % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)Bt % 16 == 0;
-  return b && (cv ? cv->iC % 4 == 0 && cv->ldx % 4 == 0 : lda % 4 == 0 && sa % 4 == 0);
+  // 32-bit byte offsets within a tile's 64 rows (a convolution's: within the
+  // images that 64 output pixels touch), below the out-of-range offset 2^31
+  const long rows = 64 * 4, lim = 0x7fffffffL;
+  if (!b || long(ldb) * rows > lim || ldb < 0) return false;
+  if (!cv) return lda % 4 == 0 && sa % 4 == 0 && lda >= 0 && lda * rows <= lim;
+  const long imgs = 64 / std::max(1, cv->oH * cv->oW) + 2;
+  return cv->iC % 4 == 0 && cv->ldx % 4 == 0 && imgs * cv->iH * cv->iW * cv->ldx * 4 <= lim;
 }
 
 hipError_t gemm_f32(const float *A, const float *Bt, int M, int N, int K, long lda, long ldb, int batch, long sa,
