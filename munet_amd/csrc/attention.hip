@@ -791,7 +791,10 @@ int cu_count() {
 // flash_attn_tr_kernel for this head size: one 16-row query group per wave
 // (more resident waves hide the softmax latency) up to hd 64; above, two
 // groups per wave, whose shared fragment reads balance LDS against the matrix
-// cores, once that still gives every CU a workgroup.
+// cores, once that still fills the chip: two workgroups a CU, four with the
+// causal mask, whose short query blocks end early (bf16, hd 128, one group |
+// two: 2 x 16 heads x 1000 keys 28.8 | 41.1 us causal, 38.2 | 42.4 full; 4 x 16
+// x 1024 44.0 | 45.6 and 71.0 | 57.3; 8 x 16 x 1024 76.4 | 71.2 and 130.6 | 106.9).
 template <int DT>
 hipError_t flash_tr(const void *q, const void *k, const void *v, void *ctx, int B, int H, int T, int hd, int causal,
                     float scale, int textbook, hipStream_t st) {
@@ -800,7 +803,8 @@ hipError_t flash_tr(const void *q, const void *k, const void *v, void *ctx, int 
   const long bh = long(B) * H;
   const bool p2 = hd == HD && pow2(scale);
   static const int forced = tr_rows_env();
-  const int rw = hd <= 64 ? (forced && p2 && !textbook ? forced : 1) : long((T + 127) / 128) * bh >= 256 ? 2 : 1;
+  const long wide = long((T + 127) / 128) * bh;  // workgroups of two groups per wave
+  const int rw = hd <= 64 ? (forced && p2 && !textbook ? forced : 1) : forced ? forced : wide >= (causal ? 1024 : 512) ? 2 : 1;
   const dim3 grid(unsigned(long((T + 64 * rw - 1) / (64 * rw)) * bh));
   const float c2 = (p2 ? scale : 1.0f) * 1.4426950408889634f;
 #define MH_TR(HDP, RW, TXT, P2)                                                                                    \
