@@ -1543,7 +1543,8 @@ struct mh_decoder {
   // page-locked staging of what a call moves over the bus, so that its copies
   // queue behind the kernels and one wait covers them all (each copy to or
   // from pageable memory, the error flag's among them, was a wait of its own:
-  // 52 of a step's 329 us)
+  // a step around a 250 us graph 329 us, now 318 with logits; a prompt of 60
+  // and 16 steps without 6.29 -> 5.86 ms)
   struct Pinned {
     int state[3];
     int flag;

@@ -30,9 +30,9 @@ F32, F16, BF16 = synth.F32, synth.F16, synth.BF16
                                       (2, 40, 2, 32)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_attention_textbook_core(hip, orc, dt, B, T, H, hd, causal):
-    """Textbook keys: hd 64 16-bit runs the flash kernel's row-staged K
-    variant (any T: ragged tiles are row-masked), the rest the generic
-    kernel."""
+    """Textbook keys: 16-bit heads in multiples of 8 run the flash kernel's
+    row-staged K variant (any T: ragged tiles are row-masked), fp32 its own
+    flash kernel, the rest the generic kernel."""
     E = H * hd
     q2, k2, v2 = rand((B * T, E), dt, 60), rand((B * T, E), dt, 61), rand((B * T, E), dt, 62)
     ref = orc.mha_core(q2, k2, v2, B, T, H, causal, dt, textbook=True)
