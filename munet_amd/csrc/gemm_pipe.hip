@@ -14,7 +14,7 @@ namespace {
 // Width of one wave's tile (columns) for each tile code.
 int pipe_wave_cols(int tile) {
   switch (tile) {
-  case 0: case 7: case 9: return 64;
+  case 0: case 7: case 9: case 27: return 64;
   case 3: case 8: case 10: case 11: case 17: return 48;
   case 21: case 22: case 24: return 48;
   case 26: return 16;
@@ -37,8 +37,9 @@ int pipe_wave_cols(int tile) {
 //    attention out-projection): direct-to-LDS 128x96, 4 stages, eight waves
 //    (one workgroup per CU, so deep stages and two waves per SIMD hide the
 //    memory latency; out-projection 13.9 -> 12.9 us against four waves);
-//  * up to 256 128x128 tiles: register-staged 128x128 (1500 x 2304 x 768 13.0
-//    us; 128x96 15.8, direct-to-LDS 128x128 14.0), with a GELU 128x64 (fp16:
+//  * up to 256 128x128 tiles: direct-to-LDS 128x128, eight waves and four
+//    stages (gemm_pipe_deep.hip: 2000 x 2048 x 8192 74.5 us; register-staged
+//    87.4, two stages 110, 128x64 97), with a GELU 128x64 (fp16:
 //    64x64), whose two to four workgroups per CU overlap one's epilogue with
 //    another's loop (2048 x 2048 x 512: bf16 12.1 -> 11.3 us, fp16, whose
 //    half-away roundings take more, 25.1 -> 16.3, 128x64 18.3);
@@ -65,7 +66,7 @@ int auto_tile(bool dma, int dt, int act, int M, int N, int K, int batch) {
   if (dma && M % 128 == 0 && N % 288 == 0 && t288 >= 232 && t288 <= 256) return 19;
   if (dma && N % 96 == 0 && t96 <= 256) return 17;
   if (dma && t128 > 128) {
-    if (t128 <= 256) return act != ACT_GELU ? 0 : dt == F16 ? 2 : 1;
+    if (t128 <= 256) return act != ACT_GELU ? 27 : dt == F16 ? 2 : 1;
     if (N % 96 == 0 && t96 <= 512) return 3;
     const long rem = t128 % 512;
     const double c9 = double(t128 / 512) + (rem > 256 ? 1.0 : rem > 0 ? 0.75 : 0.0);

@@ -1284,7 +1284,7 @@ hipError_t gemm_pipe_wide(int dt, int kind, int tile, const void *A, const void 
                           int batch, long sa, long sb, long sc, const EpiArgs &ep, hipStream_t st);
 // Small tiles with many stages (gemm_pipe_deep.hip), every program but
 // PK_BIAS_NT: 20 64x64, 21 64x48, 22 64x96, 23 32x64, 24 32x48, 25 128x64, 26
-// 32x32 (21 and 24: PK_BIAS_RESID_ST only; 23 and 26: no folded LayerNorm).
+// 32x32, 27 128x128 (21 and 24: PK_BIAS_RESID_ST only; 23 and 26: no folded LayerNorm).
 hipError_t gemm_pipe_deep(int dt, int kind, int tile, const void *A, const void *Bt, int M, int N, int K, long lda, long ldb,
                           int batch, long sa, long sb, long sc, const EpiArgs &ep, hipStream_t st);
 hipError_t gemm_pipe_fixed_dma(int dt, int kind, int tile, const void *A, const void *Bt, int M, int N, int K, long lda,

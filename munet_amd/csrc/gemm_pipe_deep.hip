@@ -14,7 +14,14 @@
 // nothing; K split over a workgroup's waves with fragments straight from
 // memory was slower than three stages (the MFMA operand layout puts sixteen
 // rows in each quarter of a load).
-// Tiles: 20 64x64, 21 64x48, 22 64x96, 23 32x64, 24 32x48, 25 128x64, 26 32x32.
+// 27 is the 128x128 tile of products of 129 to 256 such tiles, eight waves and
+// four stages: two waves per SIMD and three slabs in flight where the
+// register-staged four-wave tile has one of each (bf16, us: 2000 x 2048 x 8192
+// 87.4 -> 74.5, 2000 x 2048 x 2048 23.9 -> 21.8, 4096 x 1024 x 4096 44.4 -> 40.3,
+// 4096 x 1024 x 1024 15.5 -> 13.7; fp16 2000 x 2048 x 2048 28.9 -> 24.3; four waves
+// on four stages 80.6, 21.2, 40.4, 13.7 and 26.5).
+// Tiles: 20 64x64, 21 64x48, 22 64x96, 23 32x64, 24 32x48, 25 128x64, 26 32x32,
+// 27 128x128.
 #include "gemm_pipe.hpp"
 
 namespace mh {
@@ -29,6 +36,7 @@ hipError_t run(int tile, const void *A, const void *Bt, int M, int N, int K, lon
   case 20: launch_dma<DT, 64, 64, 2, 2, 8, EK>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st); break;
   case 22: launch_dma<DT, 64, 96, 2, 2, 7, EK>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st); break;
   case 25: launch_dma<DT, 128, 64, 4, 2, 6, EK>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st); break;
+  case 27: launch_dma<DT, 128, 128, 4, 2, 4, EK>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st); break;
   // 48-column wave tiles, for LayerNorm partials of 48 columns
   case 21:
     if constexpr (KT::ST) launch_dma<DT, 64, 48, 4, 1, 10, EK>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, st);

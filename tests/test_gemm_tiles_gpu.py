@@ -173,7 +173,7 @@ def test_f32_conv_columns(hip, B, iC, H, W, oC, k, s, p):
     assert float((out.cpu().double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24 + 1e-6
 
 
-@pytest.mark.parametrize("tile", list(range(220, 227)))
+@pytest.mark.parametrize("tile", list(range(220, 228)))
 def test_deep_tiles(tile, hip, orc, monkeypatch):
     """The small many-stage tiles (up to 16 stages: products of fewer slabs
     than stages re-load the last one) at the edges of test_forced_tile's shapes
@@ -183,7 +183,7 @@ def test_deep_tiles(tile, hip, orc, monkeypatch):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (33, 96, 128), (256, 1024, 64), (257, 1024, 64), (500, 2048, 192), (512, 768, 256),
-                                   (2048, 768, 64), (2049, 768, 64), (300, 4096, 64)])
+                                   (2048, 768, 64), (2049, 768, 64), (300, 4096, 64), (1900, 2056, 128), (4096, 1024, 192)])
 def test_deep_tile_choice_bits(M, N, K, hip, monkeypatch):
     """Both sides of each border of the small-tile choice (at most one tile per
     CU) give the 128x128 kernel's bits, bias + GELU and bias + residual."""

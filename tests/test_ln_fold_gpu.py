@@ -140,7 +140,7 @@ def test_decoder_fold_partial_counts_vs_oracle(orc, d, heads):
     _argmax_check(y, ref, synth.BF16)
 
 
-@pytest.mark.parametrize("tile", [str(t) for t in range(220, 227)])
+@pytest.mark.parametrize("tile", [str(t) for t in range(220, 228)])
 def test_folded_decoder_bit_identical_on_deep_tiles(monkeypatch, tile):
     """The small many-stage tiles: every program of the folded decoder (a tile
     without the program's form takes 64x64) gives the automatic choice's bits."""
