@@ -25,10 +25,9 @@
 // Contiguous same-shape operands take a vectorised path (8 values per thread
 // per step, 16-byte loads for 16-bit types); all kernels are grid-stride and
 // sized to a few waves per CU.
-#include <algorithm>
-
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
+#include "launch_shapes.hpp"
 
 namespace mh {
 
@@ -157,22 +156,22 @@ binary_row_vec_kernel(const uint4 *__restrict__ a, const uint4 *__restrict__ b, 
   if (ry >= rpb || c >= cpr) return;
   float bv[V::E];
   V::dec(b[c], bv);
-  constexpr int U = 4;
-  const int step = gridDim.x * rpb;
-  for (int r = blockIdx.x * rpb + ry; r < rows; r += U * step) {
+  constexpr int U = kRowsInFlight;
+  const long step = long(gridDim.x) * rpb;
+  walk_rows(long(blockIdx.x) * rpb + ry, U * step, rows, [&](long r) {
     uint4 q[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) q[u] = a[size_t(min(long(r) + long(u) * step, long(rows) - 1)) * cpr + c];
+    for (int u = 0; u < U; ++u) q[u] = a[min(r + u * step, long(rows) - 1) * cpr + c];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (long(r) + long(u) * step >= rows) break;
+      if (r + u * step >= rows) break;
       float x[V::E];
       V::dec(q[u], x);
 #pragma unroll
       for (int e = 0; e < V::E; ++e) x[e] = binop(OP, x[e], bv[e]);
-      o[(size_t(r) + size_t(u) * step) * cpr + c] = V::enc(x);
+      o[(r + u * step) * cpr + c] = V::enc(x);
     }
-  }
+  });
 }
 
 template <int DT>
@@ -513,16 +512,14 @@ hipError_t binary(int dt, int op, const void *a, const void *b, void *out, const
   }
   if (row_bcast && !contig && cols % int(per) == 0 && g.total / cols < 0x7fffffff && (uintptr_t)a % 16 == 0 &&
       (uintptr_t)b % 16 == 0 && (uintptr_t)out % 16 == 0 && (dt == F32 || dt == F16 || dt == BF16)) {
-    const int rows = int(g.total / cols), cpr = cols / int(per), tpr = std::min(cpr, 256), rpb = 256 / tpr;
-    // up to 8192 workgroups, a thread with four rows in flight
-    const int gy = (cpr + tpr - 1) / tpr;
-    const int gx = std::max(1, std::min((rows + 4 * rpb - 1) / (4 * rpb), 8192 / gy));
-    if (gy <= 65535) {
-      const dim3 grid(gx, gy);
+    const int rows = int(g.total / cols), cpr = cols / int(per);
+    const RowBcastShape rs = row_bcast_shape(rows, cpr);
+    if (rs.gy <= 65535) {
+      const dim3 grid(rs.gx, rs.gy);
       const uint4 *a4 = static_cast<const uint4 *>(a), *b4 = static_cast<const uint4 *>(b);
       uint4 *o4 = static_cast<uint4 *>(out);
 #define MH_BR(DTV, OPV) \
-  hipLaunchKernelGGL((binary_row_vec_kernel<DTV, OPV>), grid, dim3(256), 0, st, a4, b4, o4, rows, cpr, tpr)
+  hipLaunchKernelGGL((binary_row_vec_kernel<DTV, OPV>), grid, dim3(256), 0, st, a4, b4, o4, rows, cpr, rs.tpr)
 #define MH_BROP(DTV)                                                                                         \
   switch (op) {                                                                                              \
   case BIN_ADD: MH_BR(DTV, BIN_ADD); break;                                                                  \

@@ -1,0 +1,48 @@
+// Host run of csrc/launch_shapes.hpp over row counts up to the largest that
+// the calls admit (tests/test_launch_shapes.py compiles and runs it under the
+// undefined-behaviour sanitizer).  Prints "ok" or the first fault.
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "launch_shapes.hpp"
+
+static void fail(const char *what, long a, long b, long c) {
+  std::printf("%s: %ld %ld %ld\n", what, a, b, c);
+  std::exit(1);
+}
+
+// Every row that any thread of the row-broadcast launch loads or stores.
+static void row_bcast(long rows, int cpr) {
+  const mh::RowBcastShape s = mh::row_bcast_shape(rows, cpr);
+  if (s.tpr < 1 || s.rpb < 1 || s.gx < 1 || s.gy < 1 || s.gx > 8192 || s.tpr * s.gy < cpr) fail("shape", rows, cpr, s.gx);
+  const long step = long(s.gx) * s.rpb, U = mh::kRowsInFlight;
+  const bool all = rows <= 100000;
+  std::vector<int> seen(all ? rows : 0, 0);
+  auto thread = [&](long first) {
+    long trips = 0, last = -1;
+    mh::walk_rows(first, U * step, rows, [&](long r) {
+      if (r < 0 || r >= rows || r <= last || ++trips > rows) fail("row", rows, cpr, r);
+      last = r;
+      for (long u = 0; u < U; ++u)
+        if (all && r + u * step < rows) ++seen[r + u * step];
+    });
+    const long want = first < rows ? (rows - first + U * step - 1) / (U * step) : 0;
+    if (trips != want) fail("trips", rows, first, trips);
+  };
+  if (all) {
+    for (long f = 0; f < step; ++f) thread(f);
+    for (long r = 0; r < rows; ++r)
+      if (seen[r] != 1) fail("covered", rows, r, seen[r]);
+  } else {
+    for (long f : {0L, step / 2, step - 1}) thread(f);
+  }
+}
+
+int main() {
+  const long rows[] = {1, 2, 3, 5, 255, 1024, 1025, 65537, 99999, 8388609, 2139095040, 2139095041, 2147483000, 2147483646};
+  for (long r : rows)
+    for (int cpr : {1, 2, 3, 8, 100, 255, 256, 257, 5000, 3000000})
+      if (r * cpr < (1L << 35)) row_bcast(r, cpr);  // 512 GiB operands and below
+  std::printf("ok\n");
+}
