@@ -466,8 +466,10 @@ hipError_t argmax_dt(const void *x, int32_t *out, int rows, int cols, long ld, h
     if (vec) hipLaunchKernelGGL((argmax_kernel<DT, 64, true>), dim3(rows), dim3(64), 0, st, X, out, cols, ld);
     else hipLaunchKernelGGL((argmax_kernel<DT, 64, false>), dim3(rows), dim3(64), 0, st, X, out, cols, ld);
   } else {
-    if (vec) hipLaunchKernelGGL((argmax_kernel<DT, 1024, true>), dim3(rows), dim3(1024), 0, st, X, out, cols, ld);
-    else hipLaunchKernelGGL((argmax_kernel<DT, 1024, false>), dim3(rows), dim3(1024), 0, st, X, out, cols, ld);
+    split_rows(rows, 1024, [&](long r, int n) {
+      if (vec) hipLaunchKernelGGL((argmax_kernel<DT, 1024, true>), dim3(n), dim3(1024), 0, st, X + r * ld, out + r, cols, ld);
+      else hipLaunchKernelGGL((argmax_kernel<DT, 1024, false>), dim3(n), dim3(1024), 0, st, X + r * ld, out + r, cols, ld);
+    });
   }
   return hipGetLastError();
 }

@@ -15,6 +15,13 @@ __host__ __device__ __forceinline__ void walk_rows(long first, long step, long r
   for (long r = first; r < rows; r += step) f(r);
 }
 
+// f(row0, n) for the launches that cover rows with one workgroup of `threads`
+// per row: a launch's work-items must fit in 32 bits.
+template <class F> inline void split_rows(long rows, int threads, F f) {
+  const long cap = 0xffffffffL / threads;
+  for (long r = 0; r < rows; r += cap) f(r, int(std::min(cap, rows - r)));
+}
+
 // Row-broadcast kernel: tpr threads per row, rpb rows per 256-thread
 // workgroup, gx x gy workgroups for rows of cpr 16-byte chunks; up to 8192
 // workgroups, a thread with kRowsInFlight rows in flight.

@@ -13,6 +13,7 @@
 // arithmetic on decoded values with one rounding at the output.
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
+#include "launch_shapes.hpp"
 
 namespace mh {
 
@@ -306,20 +307,26 @@ hipError_t softmax_dt(const void *x, void *y, int rows, int cols, hipStream_t st
   const T *X = (const T *)x;
   T *Y = (T *)y;
   const bool vec = cols % 4 == 0 && (uintptr_t)x % (4 * sizeof(T)) == 0 && (uintptr_t)y % (4 * sizeof(T)) == 0;
-#define MH_SM(TH, N)                                                                                                  \
+#define MH_SM1(TH, N, X, Y, R)                                                                                        \
   {                                                                                                                   \
-    const dim3 g(TH == 64 ? (rows + 3) / 4 : rows), b(TH == 64 ? 256 : TH);                                           \
-    if (vec) hipLaunchKernelGGL((softmax_row_kernel<DT, TH, N / 4, 4>), g, b, 0, st, X, Y, rows, cols);               \
-    else hipLaunchKernelGGL((softmax_row_kernel<DT, TH, N, 1>), g, b, 0, st, X, Y, rows, cols);                       \
+    const dim3 g(TH == 64 ? (R + 3) / 4 : R), b(TH == 64 ? 256 : TH);                                                 \
+    if (vec) hipLaunchKernelGGL((softmax_row_kernel<DT, TH, N / 4, 4>), g, b, 0, st, X, Y, R, cols);                  \
+    else hipLaunchKernelGGL((softmax_row_kernel<DT, TH, N, 1>), g, b, 0, st, X, Y, R, cols);                          \
   }
-  if (cols <= 256) MH_SM(64, 4)
-  else if (cols <= 512) MH_SM(64, 8)
+#define MH_SM(TH, N)                                                                                                  \
+  split_rows(rows, TH, [&](long r, int n) { MH_SM1(TH, N, X + r * cols, Y + r * cols, n) });
+  if (cols <= 256) MH_SM1(64, 4, X, Y, rows)
+  else if (cols <= 512) MH_SM1(64, 8, X, Y, rows)
   else if (cols <= 2048) MH_SM(256, 8)
   else if (cols <= 4096) MH_SM(256, 16)
   else if (cols <= 8192) MH_SM(1024, 8)
   else if (cols <= 16384) MH_SM(1024, 16)
-  else hipLaunchKernelGGL((softmax_long_kernel<DT>), dim3(rows), dim3(1024), 0, st, X, Y, cols);
+  else
+    split_rows(rows, 1024, [&](long r, int n) {
+      hipLaunchKernelGGL((softmax_long_kernel<DT>), dim3(n), dim3(1024), 0, st, X + r * cols, Y + r * cols, cols);
+    });
 #undef MH_SM
+#undef MH_SM1
   return hipGetLastError();
 }
 

@@ -39,10 +39,22 @@ static void row_bcast(long rows, int cpr) {
   }
 }
 
+// The launches of one workgroup per row: consecutive, all rows, 32-bit sizes.
+static void split(long rows, int threads) {
+  long next = 0;
+  mh::split_rows(rows, threads, [&](long r, int n) {
+    if (r != next || n < 1 || long(n) * threads > 0xffffffffL) fail("launch", rows, r, n);
+    next = r + n;
+  });
+  if (next != rows) fail("rows", rows, threads, next);
+}
+
 int main() {
   const long rows[] = {1, 2, 3, 5, 255, 1024, 1025, 65537, 99999, 8388609, 2139095040, 2139095041, 2147483000, 2147483646};
   for (long r : rows)
     for (int cpr : {1, 2, 3, 8, 100, 255, 256, 257, 5000, 3000000})
       if (r * cpr < (1L << 35)) row_bcast(r, cpr);  // 512 GiB operands and below
+  for (long r : {1L, 67108863L, 4194303L, 4194304L, 16777216L, 67108864L, 2147483647L})
+    for (int threads : {256, 1024}) split(r, threads);
   std::printf("ok\n");
 }

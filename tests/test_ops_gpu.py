@@ -431,6 +431,30 @@ def test_argmax_rows(hip, dt, cols):
     assert np.array_equal(to_host(out, I32), ref)
 
 
+def test_many_long_rows(hip):
+    """More rows than one launch of a workgroup per row can hold (1024 threads
+    from 1025 columns of an argmax on, 256 of a softmax to 4096): the rows on
+    both sides of the launch border.  Softmax rows are one value high among
+    -inf, so exactly 0 and 1."""
+    import torch
+    rows, cols = 2 ** 22 + 1, 1032
+    x = torch.zeros(rows, cols, dtype=torch.bfloat16, device="cuda")
+    at = torch.randint(0, cols, (rows,), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    x.scatter_(1, at.view(-1, 1), 1.0)
+    out = empty((rows,), I32)
+    hip.argmax(x, out, rows, cols)
+    assert torch.equal(out, at.int())
+    del x
+    rows, cols = 2 ** 24 + 1, 516
+    x = torch.full((rows, cols), -float("inf"), dtype=torch.bfloat16, device="cuda")
+    at = torch.arange(rows, device="cuda") % cols
+    x.scatter_(1, at.view(-1, 1), 1.0)
+    y = torch.empty_like(x)
+    hip.softmax(x, y, rows, cols)
+    x.fill_(0.0).scatter_(1, at.view(-1, 1), 1.0)
+    assert all(torch.equal(y[i:i + 2 ** 20], x[i:i + 2 ** 20]) for i in range(0, rows, 2 ** 20))
+
+
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("B,iC,H,W,oC,k,s,p", [(2, 3, 9, 9, 4, 3, 1, 1), (2, 3, 9, 9, 4, 3, 2, 1),
                                                (1, 16, 12, 10, 32, 3, 1, 1), (2, 8, 8, 8, 16, 1, 1, 0),
