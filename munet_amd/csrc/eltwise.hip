@@ -25,6 +25,8 @@
 // Contiguous same-shape operands take a vectorised path (8 values per thread
 // per step, 16-byte loads for 16-bit types); all kernels are grid-stride and
 // sized to a few waves per CU.
+#include <type_traits>
+
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
 #include "launch_shapes.hpp"
@@ -395,42 +397,55 @@ embedding_row16_kernel(const int32_t *__restrict__ ids, const uint16_t *__restri
   }
 }
 
-// First index of the row's maximum (NaN never wins; all-NaN rows give 0), one
-// workgroup of TH threads per row of cols values, rows ld apart: TH = 64 for
-// short rows, 1024 for a vocabulary's.  With VEC a thread takes 16-byte chunks
-// tid, tid + TH, ... (ascending, so a strict > keeps its first maximum), four
-// in flight.  A vocabulary row on one wave with one value per load was a chain
-// of 500 memory trips: 32000 bf16 values 154 us, here 5.9 (four rows in one launch).
-template <int DT, int TH, bool VEC>
-__global__ void __launch_bounds__(TH)
-argmax_kernel(const typename Store<DT>::T *__restrict__ x, int32_t *__restrict__ out, int cols, long ld) {
+// First index of the row's maximum (NaN never wins; all-NaN rows give 0), TH
+// threads per row (four rows per workgroup for TH = 64), rows ld apart.  A
+// thread takes values, with VEC 16-byte chunks, t, t + TH, ... (ascending, so
+// a strict > keeps its first maximum), U in flight; those past the row are
+// skipped, not loaded again, so that a short row costs what it holds.
+//
+// A vocabulary row on one wave with one value per load was a chain of 500
+// memory trips: 32000 bf16 values 87 us (four rows in one launch), with 1024
+// threads and chunks 4.4.  A workgroup per row for many or short rows pays its
+// reduction over 16 waves each time: 20000 rows of 1025 bf16 values 88 us
+// against 11.4 with a wave per row, 4096 of 2048 25.5 against 4.0.
+template <int DT, int TH, bool VEC, int U>
+__global__ void __launch_bounds__(TH < 256 ? 256 : TH)
+argmax_kernel(const typename Store<DT>::T *__restrict__ x, int32_t *__restrict__ out, int rows, int cols, long ld) {
   typedef Vec16<DT> V;
-  constexpr int E = VEC ? V::E : 1, U = 4;
-  __shared__ float sv[TH / 64];
-  __shared__ int si[TH / 64];
-  const typename Store<DT>::T *p = x + long(blockIdx.x) * ld;
-  const int tid = threadIdx.x, n = cols / E;
+  constexpr int E = VEC ? V::E : 1;
+  const int row = TH == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  const unsigned tid = TH == 64 ? threadIdx.x & 63 : threadIdx.x, n = unsigned(cols) / E;
+  if (row >= rows) return;  // TH = 64: whole waves, which share nothing
+  const typename Store<DT>::T *p = x + long(row) * ld;
   float best = -INFINITY;
   int bi = 0x7fffffff;
-  auto take = [&](float v, int c) {
-    if (v > best || (bi == 0x7fffffff && v == best)) {
-      best = v;
-      bi = c;
-    }
-  };
-  for (int c0 = tid; c0 < n; c0 += U * TH) {
+  // U loads c0, c0 + TH, ... (guarded: those below n), then their values
+  auto batch = [&](unsigned c0, auto guarded) {
+    constexpr bool G = decltype(guarded)::value;
     float v[U][E];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int c = min(c0 + u * TH, n - 1);  // (a repeated chunk changes nothing)
-      if constexpr (VEC) V::dec(reinterpret_cast<const uint4 *>(p)[c], v[u]);
-      else v[u][0] = Store<DT>::dec(p[c]);
+      const unsigned c = c0 + u * TH;
+      if (!G || u == 0 || c < n) {
+        if constexpr (VEC) V::dec(reinterpret_cast<const uint4 *>(p)[c], v[u]);
+        else v[u][0] = Store<DT>::dec(p[c]);
+      }
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      const unsigned c = c0 + u * TH;
+      if (!G || u == 0 || c < n)
 #pragma unroll
-      for (int e = 0; e < E; ++e) take(v[u][e], min(c0 + u * TH, n - 1) * E + e);
-  }
+        for (int e = 0; e < E; ++e)
+          if (v[u][e] > best) {
+            best = v[u][e];
+            bi = int(c * E + e);
+          }
+    }
+  };
+  unsigned c0 = tid;
+  for (; c0 + (U - 1) * TH < n; c0 += U * TH) batch(c0, std::false_type{});
+  if (c0 < n) batch(c0, std::true_type{});
   auto merge = [&](float ob, int oi) {
     if (ob > best || (ob == best && oi < bi)) {
       best = ob;
@@ -440,6 +455,8 @@ argmax_kernel(const typename Store<DT>::T *__restrict__ x, int32_t *__restrict__
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) merge(__shfl_xor(best, o, 64), __shfl_xor(bi, o, 64));
   if constexpr (TH > 64) {
+    __shared__ float sv[TH / 64];
+    __shared__ int si[TH / 64];
     if ((tid & 63) == 0) {
       sv[tid >> 6] = best;
       si[tid >> 6] = bi;
@@ -450,8 +467,15 @@ argmax_kernel(const typename Store<DT>::T *__restrict__ x, int32_t *__restrict__
     bi = tid < TH / 64 ? si[tid] : 0x7fffffff;
 #pragma unroll
     for (int o = TH / 128; o > 0; o >>= 1) merge(__shfl_xor(best, o, 64), __shfl_xor(bi, o, 64));
+    bi = __shfl(bi, 0, 64);
   }
-  if (tid == 0) out[blockIdx.x] = bi == 0x7fffffff ? 0 : bi;
+  if (bi == 0x7fffffff) {  // (wave-uniform) nothing above -inf: the first -inf
+    for (unsigned c = tid & 63; c < unsigned(cols) && bi == 0x7fffffff; c += 64)
+      if (Store<DT>::dec(p[c]) == -INFINITY) bi = int(c);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) bi = min(bi, __shfl_xor(bi, o, 64));
+  }
+  if (tid == 0) out[row] = bi == 0x7fffffff ? 0 : bi;
 }
 
 template <int DT>
@@ -459,18 +483,20 @@ hipError_t argmax_dt(const void *x, int32_t *out, int rows, int cols, long ld, h
   typedef typename Store<DT>::T T;
   const T *X = (const T *)x;
   const int e = 16 / int(sizeof(T));
-  const bool vec = cols % e == 0 && ld % e == 0 && (uintptr_t)x % 16 == 0;
-  // one wave up to 1024 values (four trips of its scalar loads), 1024 threads
-  // past it
-  if (cols <= 1024) {
-    if (vec) hipLaunchKernelGGL((argmax_kernel<DT, 64, true>), dim3(rows), dim3(64), 0, st, X, out, cols, ld);
-    else hipLaunchKernelGGL((argmax_kernel<DT, 64, false>), dim3(rows), dim3(64), 0, st, X, out, cols, ld);
-  } else {
-    split_rows(rows, 1024, [&](long r, int n) {
-      if (vec) hipLaunchKernelGGL((argmax_kernel<DT, 1024, true>), dim3(n), dim3(1024), 0, st, X + r * ld, out + r, cols, ld);
-      else hipLaunchKernelGGL((argmax_kernel<DT, 1024, false>), dim3(n), dim3(1024), 0, st, X + r * ld, out + r, cols, ld);
-    });
-  }
+  // chunks where a row has more values than a wave's lanes
+  const bool vec = cols > 64 && cols % e == 0 && ld % e == 0 && (uintptr_t)x % 16 == 0;
+  const int n = vec ? cols / e : cols, th = argmax_threads(rows, n);
+#define MH_AM(TH, U)                                                                                              \
+  split_rows(rows, TH, [&](long r, int m) {                                                                       \
+    const dim3 g(TH == 64 ? unsigned((long(m) + 3) / 4) : unsigned(m)), b(TH < 256 ? 256 : TH);                   \
+    if (vec) hipLaunchKernelGGL((argmax_kernel<DT, TH, true, U>), g, b, 0, st, X + r * ld, out + r, m, cols, ld); \
+    else hipLaunchKernelGGL((argmax_kernel<DT, TH, false, U>), g, b, 0, st, X + r * ld, out + r, m, cols, ld);    \
+  })
+  if (n <= 64) MH_AM(64, 1);
+  else if (th == 64) MH_AM(64, 4);
+  else if (th == 256) MH_AM(256, 4);
+  else MH_AM(1024, 4);
+#undef MH_AM
   return hipGetLastError();
 }
 

@@ -22,6 +22,18 @@ template <class F> inline void split_rows(long rows, int threads, F f) {
   for (long r = 0; r < rows; r += cap) f(r, int(std::min(cap, rows - r)));
 }
 
+// Threads per row of an argmax of rows of n loads (values or 16-byte chunks): a
+// wave up to 256 (four per lane), and up to 2048 where the rows alone fill the
+// chip; 1024 threads for the longest rows and for few long ones.  64 | 256 |
+// 1024 threads, bf16, us: chunks, 20000 rows of n = 256 14.9 | 20.2 | 70.8, 4096
+// of 2048 23.1 | 22.9 | 24.7, 33 of 4000 8.5 | 4.9 | 4.6, 1000 of 4000 12.7 |
+// 12.4 | 14.3; values, 4096 of 1025 3.7 | 5.9 | 17.5, 1000 of
+// 50257 68.8 | 24.1 | 19.2.
+inline int argmax_threads(long rows, int n) {
+  if (n <= 256 || (rows >= 2048 && n <= 2048)) return 64;
+  return n >= 4096 || (n >= 2048 && rows <= std::max(256, n / 8)) ? 1024 : 256;
+}
+
 // Row-broadcast kernel: tpr threads per row, rpb rows per 256-thread
 // workgroup, gx x gy workgroups for rows of cpr 16-byte chunks; up to 8192
 // workgroups, a thread with kRowsInFlight rows in flight.

@@ -54,7 +54,12 @@ int main() {
   for (long r : rows)
     for (int cpr : {1, 2, 3, 8, 100, 255, 256, 257, 5000, 3000000})
       if (r * cpr < (1L << 35)) row_bcast(r, cpr);  // 512 GiB operands and below
+  // many rows on a wave each, few long ones on a workgroup
+  const struct { long rows; int n, th; } am[] = {{20000, 1025, 64}, {4096, 2048, 64}, {4, 64, 64}, {1, 257, 256},
+                                                 {1000, 512, 256}, {4, 4000, 1024}, {4096, 4000, 256}, {1000, 50257, 1024}};
+  for (const auto &a : am)
+    if (mh::argmax_threads(a.rows, a.n) != a.th) fail("argmax", a.rows, a.n, mh::argmax_threads(a.rows, a.n));
   for (long r : {1L, 67108863L, 4194303L, 4194304L, 16777216L, 67108864L, 2147483647L})
-    for (int threads : {256, 1024}) split(r, threads);
+    for (int threads : {64, 256, 1024}) split(r, threads);
   std::printf("ok\n");
 }

@@ -408,12 +408,13 @@ def test_argmax(hip, dt):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("cols", [1, 8, 63, 1000, 1024, 1025, 4104, 32000, 40007])
-def test_argmax_rows(hip, dt, cols):
-    """Both row widths and both load widths: ties far apart give the first
-    index, NaN never wins, rows of -inf and of NaN give index 0, whole numbers
-    exactly."""
-    x = rand((6, cols), dt, 94)
+@pytest.mark.parametrize("rows,cols", [(6, c) for c in (1, 8, 63, 64, 65, 72, 257, 1000, 1024, 1025, 4104, 32000, 40007)] +
+                         [(2055, c) for c in (65, 1025, 2049, 4104)])
+def test_argmax_rows(hip, dt, rows, cols):
+    """Each thread count per row and both load widths: ties far apart give the
+    first index, NaN never wins, rows of -inf and of NaN give index 0, rows of
+    -inf and NaN the first -inf, whole numbers exactly."""
+    x = rand((rows, cols), dt, 94)
     f = dec(x, dt)
     f[1, cols // 3] = f[1, cols - 1] = 60.0
     f[2, 0] = f[2, cols // 2] = f[2, cols - 1] = 60.0
@@ -426,8 +427,11 @@ def test_argmax_rows(hip, dt, cols):
     ref[4] = 0
     odd = np.where(np.arange(cols) % 2 == 1, f[5], -np.inf)
     ref[5] = int(np.argmax(odd)) if cols > 1 else 0
-    out = empty((6,), I32)
-    hip.argmax(to_device(x, dt), out, 6, cols)
+    x[0, :] = nan
+    x[0, cols - 1 - cols // 3:] = synth.encode(np.array([-np.inf]), dt)[0]
+    ref[0] = cols - 1 - cols // 3
+    out = empty((rows,), I32)
+    hip.argmax(to_device(x, dt), out, rows, cols)
     assert np.array_equal(to_host(out, I32), ref)
 
 
