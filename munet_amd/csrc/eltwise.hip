@@ -144,11 +144,11 @@ __global__ void binary_row_kernel(const typename Store<DT>::T *__restrict__ a,
 
 // The same on whole 16-byte chunks (the host checks the alignment and cols % E
 // == 0): a thread owns one chunk column, holds its chunk of b, and walks rows
-// r, r + step, ... four in flight; the cpr chunk columns of a row are spread
+// r, r + step, ... U in flight; the cpr chunk columns of a row are spread
 // over threads and blockIdx.y, 256 / cpr rows per workgroup where a row has
 // fewer.  Bound: HBM; the one-value-per-thread kernel, with a 64-bit modulo per
-// value, took 22.9 us for 4096 x 4096 bf16 (2.9 TB/s); this one 11.7 (5.7).
-template <int DT, int OP>
+// value, took 20.7 us for 4096 x 4096 bf16 (3.2 TB/s); this one 11.4 (5.9).
+template <int DT, int OP, int U>
 __global__ void __launch_bounds__(256)
 binary_row_vec_kernel(const uint4 *__restrict__ a, const uint4 *__restrict__ b, uint4 *__restrict__ o, int rows, int cpr,
                       int tpr) {
@@ -158,7 +158,6 @@ binary_row_vec_kernel(const uint4 *__restrict__ a, const uint4 *__restrict__ b, 
   if (ry >= rpb || c >= cpr) return;
   float bv[V::E];
   V::dec(b[c], bv);
-  constexpr int U = kRowsInFlight;
   const long step = long(gridDim.x) * rpb;
   walk_rows(long(blockIdx.x) * rpb + ry, U * step, rows, [&](long r) {
     uint4 q[U];
@@ -538,16 +537,22 @@ hipError_t binary(int dt, int op, const void *a, const void *b, void *out, const
 #undef MH_BV
     return hipGetLastError();
   }
-  if (row_bcast && !contig && cols % int(per) == 0 && g.total / cols < 0x7fffffff && (uintptr_t)a % 16 == 0 &&
+  // (fp16 below 2^19 values: eight of its half-away roundings in a row cost a
+  // thread more than one value per thread, 300 x 768 2.4 us, in chunks 2.9;
+  // 2000 x 768 4.5 and 3.7)
+  if (row_bcast && !contig && !(dt == F16 && g.total < 1u << 19) && cols % int(per) == 0 && g.total / cols < 0x7fffffff && (uintptr_t)a % 16 == 0 &&
       (uintptr_t)b % 16 == 0 && (uintptr_t)out % 16 == 0 && (dt == F32 || dt == F16 || dt == BF16)) {
     const int rows = int(g.total / cols), cpr = cols / int(per);
-    const RowBcastShape rs = row_bcast_shape(rows, cpr);
+    const RowBcastShape rs = row_bcast_shape(rows, cpr, dt == F16);
     if (rs.gy <= 65535) {
       const dim3 grid(rs.gx, rs.gy);
       const uint4 *a4 = static_cast<const uint4 *>(a), *b4 = static_cast<const uint4 *>(b);
       uint4 *o4 = static_cast<uint4 *>(out);
-#define MH_BR(DTV, OPV) \
-  hipLaunchKernelGGL((binary_row_vec_kernel<DTV, OPV>), grid, dim3(256), 0, st, a4, b4, o4, rows, cpr, rs.tpr)
+#define MH_BR(DTV, OPV)                                                                                       \
+  if (rs.u == 1)                                                                                             \
+    hipLaunchKernelGGL((binary_row_vec_kernel<DTV, OPV, 1>), grid, dim3(256), 0, st, a4, b4, o4, rows, cpr, rs.tpr); \
+  else                                                                                                       \
+    hipLaunchKernelGGL((binary_row_vec_kernel<DTV, OPV, kRowsInFlight>), grid, dim3(256), 0, st, a4, b4, o4, rows, cpr, rs.tpr)
 #define MH_BROP(DTV)                                                                                         \
   switch (op) {                                                                                              \
   case BIN_ADD: MH_BR(DTV, BIN_ADD); break;                                                                  \

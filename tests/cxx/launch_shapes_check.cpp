@@ -13,10 +13,13 @@ static void fail(const char *what, long a, long b, long c) {
 }
 
 // Every row that any thread of the row-broadcast launch loads or stores.
-static void row_bcast(long rows, int cpr) {
-  const mh::RowBcastShape s = mh::row_bcast_shape(rows, cpr);
-  if (s.tpr < 1 || s.rpb < 1 || s.gx < 1 || s.gy < 1 || s.gx > 8192 || s.tpr * s.gy < cpr) fail("shape", rows, cpr, s.gx);
-  const long step = long(s.gx) * s.rpb, U = mh::kRowsInFlight;
+static void row_bcast(long rows, int cpr, bool f16) {
+  const mh::RowBcastShape s = mh::row_bcast_shape(rows, cpr, f16);
+  if (s.tpr < 1 || s.rpb < 1 || s.gx < 1 || s.gy < 1 || s.gx > 32768 || s.tpr * s.gy < cpr) fail("shape", rows, cpr, s.gx);
+  // one row per thread until the chip is full
+  if (rows * cpr < 1 << 20 && (s.u != 1 || long(s.gx) * s.rpb < std::min(rows, 32768L * s.rpb / s.gy - s.rpb)))
+    fail("rows in flight", rows, cpr, s.u);
+  const long step = long(s.gx) * s.rpb, U = s.u;
   const bool all = rows <= 100000;
   std::vector<int> seen(all ? rows : 0, 0);
   auto thread = [&](long first) {
@@ -53,7 +56,10 @@ int main() {
   const long rows[] = {1, 2, 3, 5, 255, 1024, 1025, 65537, 99999, 8388609, 2139095040, 2139095041, 2147483000, 2147483646};
   for (long r : rows)
     for (int cpr : {1, 2, 3, 8, 100, 255, 256, 257, 5000, 3000000})
-      if (r * cpr < (1L << 35)) row_bcast(r, cpr);  // 512 GiB operands and below
+      if (r * cpr < (1L << 35)) {  // 512 GiB operands and below
+        row_bcast(r, cpr, false);
+        row_bcast(r, cpr, true);
+      }
   // many rows on a wave each, few long ones on a workgroup
   const struct { long rows; int n, th; } am[] = {{20000, 1025, 64}, {4096, 2048, 64}, {4, 64, 64}, {1, 257, 256},
                                                  {1000, 512, 256}, {4, 4000, 1024}, {4096, 4000, 256}, {1000, 50257, 1024}};

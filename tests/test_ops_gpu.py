@@ -243,11 +243,12 @@ def test_softmax(hip, orc, dt, rows, cols):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("rows,cols", [(1, 8), (5, 16), (3, 2056), (700, 40), (33, 2048), (9, 4104), (2, 12), (300, 1), (4, 9)])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (5, 16), (3, 2056), (700, 40), (33, 2048), (9, 4104), (2, 12), (300, 1), (4, 9),
+                                       (65543, 8), (130, 4104), (40003, 72), (3001, 4104)])
 def test_row_broadcast_chunks(hip, orc, dt, rows, cols):
     """[rows, cols] op [cols]: the 16-byte-chunk kernel (rows narrower and
-    wider than a workgroup, row counts that are no multiple of its step) and
-    the scalar one (odd widths, and a row that starts off a 16-byte boundary)
+    wider than a workgroup, row counts that are no multiple of its step, one
+    row and four in flight per thread; fp16 from 2^19 values on) and the scalar one (odd widths, and a row that starts off a 16-byte boundary)
     against the oracle, bit for bit (one rounding of the same float op)."""
     a, b = rand((rows, cols), dt, 12), rand((cols,), dt, 13)
     info = BroadcastInfo(*compute_broadcast((rows, cols), contiguous_strides((rows, cols)), (cols,), [1]))
