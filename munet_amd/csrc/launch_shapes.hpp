@@ -57,4 +57,20 @@ inline RowBcastShape row_bcast_shape(long rows, int cpr, bool f16) {
   return s;
 }
 
+// Whether a batch of transposes takes one workgroup per slice (slices of at most
+// transpose_flat_max values with fewer than 16 rows or columns) instead of
+// 64x64 tiles, `es` bytes a value, `vec` where the tiles load and store chunks.
+// A slice takes its workgroup about 2.1 us + 0.17 ns per byte, the tiles 2.3 to
+// 4.3 us + 1.2 ns per tile over the whole batch (slices | tiles, fp32, us: 32 of
+// 64 x 9 2.4 | 4.1, 2 of 8 x 1000 7.3 | 2.4, 2 of 1 x 8000 7.7 | 3.4, 128 of them 8.6 |
+// 21.2, 128 of 3 x 1024 4.4 | 4.8, 64 of 512 x 15 7.9 | 4.6, 512 of them 10.7 |
+// 14.9; bf16 32 of 3 x 1024 3.4 | 3.2, 512 of 8 x 1000 7.5 | 6.8).
+constexpr int transpose_flat_max = 8192;
+inline bool transpose_flat(long batch, long rows, long cols, int es, bool vec) {
+  const long n = rows * cols, tiles = batch * ((rows + 63) / 64) * ((cols + 63) / 64);
+  if (batch <= 1 || (rows >= 16 && cols >= 16) || n > transpose_flat_max) return false;
+  // (a launch of tiles holds at most 65535 slices)
+  return n <= 1024 || batch > 65535 || (!vec && n * es <= 4096 + 7 * tiles);
+}
+
 }  // namespace mh

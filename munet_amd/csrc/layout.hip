@@ -17,6 +17,7 @@
 // write side are coalesced.
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
+#include "launch_shapes.hpp"
 
 namespace mh {
 
@@ -109,8 +110,8 @@ transpose_kernel(const T *__restrict__ in, T *__restrict__ out, int rows, int co
 // Slices of at most kFlat values with fewer than 16 rows or columns (a
 // convolution's [iC, kH kW] weights: 9 of a tile's 64 columns): one workgroup
 // per slice reads it as it lies into LDS and writes it in output order, both
-// coalesced.  128 slices of 64 x 9 floats 7.7 -> 4.4 us.
-constexpr int kFlat = 8192;
+// coalesced.  128 slices of 64 x 9 floats 5.1 -> 2.5 us.
+constexpr int kFlat = transpose_flat_max;
 template <typename T>
 __global__ void __launch_bounds__(256)
 transpose_flat_kernel(const T *__restrict__ in, T *__restrict__ out, int rows, int cols) {
@@ -208,12 +209,12 @@ hipError_t transpose_t(const void *in, void *out, int batch, int rows, int cols,
   constexpr int V = 16 / int(sizeof(T));
   const T *I = (const T *)in;
   T *O = (T *)out;
-  if ((rows < 16 || cols < 16) && long(rows) * cols <= kFlat && batch > 1) {
+  const bool vl = cols % V == 0 && (uintptr_t)in % 16 == 0, vs = rows % V == 0 && (uintptr_t)out % 16 == 0;
+  if (transpose_flat(batch, rows, cols, int(sizeof(T)), vl && vs)) {
     hipLaunchKernelGGL(transpose_flat_kernel<T>, dim3(batch), dim3(256), 0, st, I, O, rows, cols);
     return hipGetLastError();
   }
   const dim3 grid((cols + 63) / 64, (rows + 63) / 64, batch), block(256);
-  const bool vl = cols % V == 0 && (uintptr_t)in % 16 == 0, vs = rows % V == 0 && (uintptr_t)out % 16 == 0;
   if (vl && vs) hipLaunchKernelGGL((transpose_kernel<T, true, true>), grid, block, 0, st, I, O, rows, cols);
   else if (vl) hipLaunchKernelGGL((transpose_kernel<T, true, false>), grid, block, 0, st, I, O, rows, cols);
   else if (vs) hipLaunchKernelGGL((transpose_kernel<T, false, true>), grid, block, 0, st, I, O, rows, cols);

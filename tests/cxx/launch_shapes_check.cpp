@@ -65,6 +65,13 @@ int main() {
                                                  {1000, 512, 256}, {4, 4000, 1024}, {4096, 4000, 256}, {1000, 50257, 1024}};
   for (const auto &a : am)
     if (mh::argmax_threads(a.rows, a.n) != a.th) fail("argmax", a.rows, a.n, mh::argmax_threads(a.rows, a.n));
+  // few long slices in tiles, many or short ones flat
+  const struct { long b, r, c; int es; bool vec, flat; } tr[] = {
+      {128, 64, 9, 4, false, true}, {2, 8, 1000, 4, true, false}, {3, 1, 8000, 4, false, false}, {128, 1, 8000, 4, false, true},
+      {4, 15, 400, 4, false, false}, {2, 8, 1000, 2, true, false}, {1, 64, 9, 4, false, false}, {512, 16, 16, 4, false, false},
+      {70000, 2, 1000, 4, true, true}};
+  for (const auto &t : tr)
+    if (mh::transpose_flat(t.b, t.r, t.c, t.es, t.vec) != t.flat) fail("transpose", t.b, t.r, t.c);
   for (long r : {1L, 67108863L, 4194303L, 4194304L, 16777216L, 67108864L, 2147483647L})
     for (int threads : {64, 256, 1024}) split(r, threads);
   std::printf("ok\n");

@@ -605,12 +605,14 @@ def test_pool_upsample_concat(hip, orc, dt):
 
 @pytest.mark.parametrize("dt", [F32, BF16, I32])
 @pytest.mark.parametrize("batch,rows,cols", [(1, 64, 64), (2, 65, 72), (2, 72, 65), (3, 8, 8), (1, 9, 200), (2, 128, 9), (3, 15, 130),
-                                             (2, 1000, 9), (1, 200, 100), (1, 1, 5), (2, 24, 1000), (1, 1000, 24), (2, 130, 63)])
+                                             (2, 1000, 9), (1, 200, 100), (1, 1, 5), (2, 24, 1000), (1, 1000, 24), (2, 130, 63),
+                                             (150, 3, 1001), (130, 1001, 3)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_transpose2d(hip, dt, batch, rows, cols, shift):
     """Chunked and scalar loads and stores (lengths that are multiples of a
     16-byte chunk or not, storages that start on a boundary or one value off
-    it), ragged tiles, and the flat path of narrow slices: exact, and nothing
+    it), ragged tiles, and the flat path of narrow slices, short ones and many
+    long ones: exact, and nothing
     written past the output."""
     x = rand((batch, rows, cols), dt, 131) if dt != I32 else np.arange(batch * rows * cols, dtype=np.int32).reshape(batch, rows, cols)
     n = x.size
