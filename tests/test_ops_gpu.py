@@ -262,7 +262,7 @@ def test_row_broadcast_chunks(hip, orc, dt, rows, cols):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("cols", [1, 5, 256, 260, 513, 2049, 4096, 4100, 8193, 16384, 16385, 30001])
+@pytest.mark.parametrize("cols", [1, 5, 64, 65, 128, 132, 256, 260, 513, 2049, 4096, 4100, 8193, 16384, 16385, 30001])
 def test_softmax_rows(hip, dt, cols):
     """Each thread count per row at its edges, aligned and odd lengths, rows
     that fill no workgroup; -inf entries give exactly zero, a row with NaN,
