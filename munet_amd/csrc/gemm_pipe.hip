@@ -6,6 +6,7 @@
 // gemm_pipe_wide.hip.
 #include <algorithm>
 #include "gemm_pipe.hpp"
+#include "gemm_tiles.hpp"
 
 namespace mh {
 
@@ -24,60 +25,9 @@ int pipe_wave_cols(int tile) {
   }
 }
 
-// Automatic block tile, measured on MI355X inside the decoder forward
-// (K = 768 / 3072, M = 4096):
-//  * M tiling evenly by 256 and N by 192 into 232..256 tiles (FFN up: 256):
-//    direct-to-LDS 256x192 with eight waves, one workgroup per CU (FFN up
-//    33.1 -> 31.1 us; QKV, 192 tiles, 28.3 -> 29.5 us, so it stays below);
-//  * M tiling by 128 and N by 288 into 232..256 tiles (QKV, 4096 x 2304):
-//    direct-to-LDS 128x288, eight waves of 32x144, one workgroup per CU
-//    (forward 1.620 -> 1.609 ms against the register-staged 128x96, whose
-//    768 tiles take three rounds of two workgroups per CU);
-//  * N tiling evenly by 96 with at most one tile per CU (N = 768: FFN down,
-//    attention out-projection): direct-to-LDS 128x96, 4 stages, eight waves
-//    (one workgroup per CU, so deep stages and two waves per SIMD hide the
-//    memory latency; out-projection 13.9 -> 12.9 us against four waves);
-//  * up to 256 128x128 tiles: direct-to-LDS 128x128, eight waves and four
-//    stages (gemm_pipe_deep.hip: 2000 x 2048 x 8192 74.5 us; register-staged
-//    87.4, two stages 110, 128x64 97), with a GELU 128x64 (fp16:
-//    64x64), whose two to four workgroups per CU overlap one's epilogue with
-//    another's loop (2048 x 2048 x 512: bf16 12.1 -> 11.3 us, fp16, whose
-//    half-away roundings take more, 25.1 -> 16.3, 128x64 18.3);
-//  * N tiling by 96 into at most two 128x96 tiles per CU: register-staged
-//    128x96 (8192 x 768 x 3072 49.8 us; direct-to-LDS 128x128 55);
-//  * else the direct-to-LDS tile with the least rounds times round time: two
-//    128x128 (two stages) per CU, 256x192 and (whole tiles only) 128x288 one
-//    per CU, a round of 256x192 taking 1.25 to 1.39 and of 128x288 1.15 to 1.25
-//    of a 128x128 round, a last round of at most one 128x128 per CU 0.75 (2000 x 4096 x 1024:
-//    128x128 21.7 us, 256x192 26.8, register-staged 128x64 29.9; 2048 x 5000 x
-//    512: 22.6, 18.7, 22.0; 8192 x 2304 x 768: 50.6, 48.4, 128x288 43.6);
-//  * K % 64 != 0, register-staged: 128x128 when N tiles evenly by 128 and there
-//    are >= 2.5 tiles per CU, 128x96 when N tiles evenly by 96, else 128x128 /
-//    128x64 / 64x64 by tile count.
-// (The vocabulary head, a non-temporal output, takes direct-to-LDS 128x128
-// with two stages: see launch_dt.)
-int auto_tile(bool dma, int dt, int act, int M, int N, int K, int batch) {
-  const long t128 = long((M + 127) / 128) * ((N + 127) / 128) * batch;
-  const long t96 = long((M + 127) / 128) * ((N + 95) / 96) * batch;
-  const long t64 = long((M + 127) / 128) * ((N + 63) / 64) * batch;
-  const long t192w = long(M / 256) * (N / 192) * batch;
-  if (dma && M % 256 == 0 && N % 192 == 0 && t192w >= 232 && t192w <= 256) return 16;
-  const long t288 = long(M / 128) * (N / 288) * batch;
-  if (dma && M % 128 == 0 && N % 288 == 0 && t288 >= 232 && t288 <= 256) return 19;
-  if (dma && N % 96 == 0 && t96 <= 256) return 17;
-  if (dma && t128 > 128) {
-    if (t128 <= 256) return act != ACT_GELU ? 27 : dt == F16 ? 2 : 1;
-    if (N % 96 == 0 && t96 <= 512) return 3;
-    const long rem = t128 % 512;
-    const double c9 = double(t128 / 512) + (rem > 256 ? 1.0 : rem > 0 ? 0.75 : 0.0);
-    const long n16 = long((M + 255) / 256) * ((N + 191) / 192) * batch;
-    const double c16 = 1.33 * double((n16 + 255) / 256);
-    const double c19 = M % 128 == 0 && N % 288 == 0 ? 1.15 * double((t288 + 255) / 256) : 1e30;
-    return c9 <= c16 && c9 <= c19 ? 9 : c16 <= c19 ? 16 : 19;
-  }
-  if (N % 128 == 0 && t128 >= 640) return 0;
-  if (N % 96 == 0) return 3;
-  return (t128 >= 640 || (K >= 2048 && t128 >= 128)) ? 0 : (t64 >= 256 ? 1 : 2);
+// Automatic block tile (gemm_tiles.hpp).
+int block_tile(bool dma, int dt, const EpiArgs &ep, int M, int N, int K, int batch) {
+  return auto_tile(dma, dt == F16, ep.act == ACT_GELU ? TILE_GELU : ep.resid ? TILE_RESID : TILE_PLAIN, M, N, K, batch);
 }
 
 // Small tiles with many stages (gemm_pipe_deep.hip) while they give at most
@@ -147,9 +97,9 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // 20-31 us)
   if (tile < 0 && ep.mode == EPI_CONVT) tile = 2;
   if (tile < 0 && dma) tile = deep_tile(kind, M, N, batch, ep);
-  if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = auto_tile(dma, DT, ep.act, M, N, K, batch);
+  if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = block_tile(dma, DT, ep, M, N, K, batch);
   if (tile >= 7 && !dma) tile = 0;
-  if (tile == 19 && (M % 128 || N % 288)) tile = auto_tile(dma, DT, ep.act, M, N, K, batch);
+  if (tile == 19 && (M % 128 || N % 288)) tile = block_tile(dma, DT, ep, M, N, K, batch);
   // LayerNorm partials of stats_cols columns need wave tiles that cover whole
   // groups: move to the nearest tile whose wave-tile width is a multiple
   if (ep.stats_out && pipe_wave_cols(tile) % ep.stats_cols)

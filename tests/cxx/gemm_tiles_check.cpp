@@ -1,0 +1,38 @@
+// Host run of csrc/gemm_tiles.hpp (tests/test_launch_shapes.py): tiles that
+// were measured well ahead of the ones they displaced, and a defined choice
+// over the range.  Prints "ok" or the first fault.
+#include <cstdio>
+#include <initializer_list>
+
+#include "gemm_tiles.hpp"
+
+using namespace mh;
+
+int main() {
+  // the tile chosen is one of `a` and `b` (within the runs' noise of each other)
+  const struct { bool f16; TileEpi epi; int M, N, K, a, b; } want[] = {
+      {false, TILE_GELU, 2048, 2048, 8192, 27, 27}, {false, TILE_GELU, 500, 8192, 2048, 27, 27},
+      {false, TILE_GELU, 1100, 3072, 768, 27, 27},  {true, TILE_GELU, 2000, 2048, 8192, 27, 27},
+      {true, TILE_GELU, 2048, 2048, 512, 2, 2},     {true, TILE_GELU, 1100, 5000, 512, 1, 2},
+      {true, TILE_GELU, 8192, 4096, 512, 1, 1},     {true, TILE_GELU, 8192, 8192, 2048, 0, 9},
+      {false, TILE_RESID, 4096, 5000, 512, 0, 9},   {false, TILE_RESID, 2000, 5000, 512, 1, 0},
+      {false, TILE_RESID, 8192, 2500, 1024, 0, 9},  {true, TILE_GELU, 8192, 2048, 8192, 9, 16}};
+  for (const auto &w : want) {
+    const int t = auto_tile(true, w.f16, w.epi, w.M, w.N, w.K, 1);
+    if (t != w.a && t != w.b) {
+      std::printf("%d x %d x %d f16 %d epi %d: tile %d\n", w.M, w.N, w.K, w.f16, w.epi, t);
+      return 1;
+    }
+  }
+  for (int M : {1, 129, 4096, 100000})
+    for (int N : {1, 288, 5000, 100000})
+      for (int K : {64, 512, 8192, 1 << 20})
+        for (int e = 0; e < 12; ++e) {
+          const int t = auto_tile(e & 1, e & 2, TileEpi(e / 4), M, N, K, 3);
+          if ((t == 19 && (M % 128 || N % 288)) || ((t >= 7) && !(e & 1))) {
+            std::printf("tile %d for %d x %d x %d\n", t, M, N, K);
+            return 1;
+          }
+        }
+  std::printf("ok\n");
+}

@@ -2,6 +2,7 @@
 // the calls admit (tests/test_launch_shapes.py compiles and runs it under the
 // undefined-behaviour sanitizer).  Prints "ok" or the first fault.
 #include <cstdio>
+#include <initializer_list>
 #include <cstdlib>
 #include <vector>
 
