@@ -124,10 +124,11 @@ __device__ __forceinline__ int swz(int r, int c) { return r * 8 + (c ^ (r & 7));
 // RW: 16-row query groups per wave.  Each wave reads the whole K and V tile
 // from LDS, HDP * 256 bytes for RW * HDP / 4 + 2 RW MFMAs of 16 cycles: at
 // hd 128 one group needs 1024 LDS cycles per CU beside 544 MFMA cycles, two
-// groups break even, so hd > 64 takes RW = 2 while that leaves a workgroup
-// per CU.  A decoder block of 2 x 1000 tokens with 16 heads of 128: 1771 us
-// with the one-wave-per-query kernel that these sizes ran on, 310 us with this
-// one; a 237-token prompt at hd 64 (no 16-byte aligned K rows): 96 -> 88 us.
+// groups break even, so hd > 64 takes RW = 2 where that still fills the chip
+// (flash_tr below).  A decoder block of 2 x 1000 tokens with 16 heads of 128
+// (RW = 1): 1773 us with the one-wave-per-query kernel that these sizes ran on,
+// 280 us with this one; a 237-token prompt's block at hd 64 (no 16-byte aligned
+// K rows): 96 -> 88 us.
 //
 // Scores: the reference rounds q.k to the dtype and multiplies by the [1]
 // scale tensor (rounded again).  With a power-of-two scale (P2: hd = 64) that
@@ -759,15 +760,15 @@ bool pow2(float x) {
   int e;
   return x > 0.f && std::frexp(x, &e) == 0.5f;
 }
+// tuning overrides, read per call (so tests can compare the kernels in one
+// process): MUNET_HIP_ATTN_RW=1 or 2, 16 or 32 query rows per wave at head
+// sizes above 64; MUNET_HIP_ATTN_KERNEL=tr keeps the single-trip flash kernel;
+// MUNET_HIP_ATTN_ORDER=0 keeps the plain heaviest-first order
 int tr_rows_env() {
-  // tuning override: 1 or 2 (16 or 32 query rows per wave)
   const char *e = std::getenv("MUNET_HIP_ATTN_RW");
   const int v = e ? std::atoi(e) : 0;
   return (v == 1 || v == 2) ? v : 0;
 }
-// tuning overrides, read per call (so tests can compare the kernels in one
-// process): MUNET_HIP_ATTN_KERNEL=tr keeps the single-trip flash kernel;
-// MUNET_HIP_ATTN_ORDER=0 keeps the plain heaviest-first order
 bool pipe_kernel_env() {
   const char *e = std::getenv("MUNET_HIP_ATTN_KERNEL");
   return !(e && std::string(e) == "tr");
@@ -802,9 +803,9 @@ hipError_t flash_tr(const void *q, const void *k, const void *v, void *ctx, int 
   uint16_t *O = (uint16_t *)ctx;
   const long bh = long(B) * H;
   const bool p2 = hd == HD && pow2(scale);
-  static const int forced = tr_rows_env();
+  const int forced = tr_rows_env();
   const long wide = long((T + 127) / 128) * bh;  // workgroups of two groups per wave
-  const int rw = hd <= 64 ? (forced && p2 && !textbook ? forced : 1) : forced ? forced : wide >= (causal ? 1024 : 512) ? 2 : 1;
+  const int rw = hd <= 64 ? 1 : forced ? forced : wide >= (causal ? 1024 : 512) ? 2 : 1;
   const dim3 grid(unsigned(long((T + 64 * rw - 1) / (64 * rw)) * bh));
   const float c2 = (p2 ? scale : 1.0f) * 1.4426950408889634f;
 #define MH_TR(HDP, RW, TXT, P2)                                                                                    \
@@ -814,9 +815,7 @@ hipError_t flash_tr(const void *q, const void *k, const void *v, void *ctx, int 
   { if (rw == 2) { if (textbook) MH_TR(HDP, 2, true, false); else MH_TR(HDP, 2, false, false); } \
     else { if (textbook) MH_TR(HDP, 1, true, false); else MH_TR(HDP, 1, false, false); } }
   if (p2) {
-    if (textbook) MH_TR(64, 1, true, true);
-    else if (rw == 2) MH_TR(64, 2, false, true);
-    else MH_TR(64, 1, false, true);
+    if (textbook) MH_TR(64, 1, true, true); else MH_TR(64, 1, false, true);
   } else if (hd <= 32) {
     if (textbook) MH_TR(32, 1, true, false); else MH_TR(32, 1, false, false);
   } else if (hd <= 64) {

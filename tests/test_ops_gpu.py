@@ -160,9 +160,8 @@ def test_attention_head_sizes(hip, dt, hd, B, H, T, causal, textbook):
     """The flash kernels over head sizes (each rounded size 32 / 64 / 96 / 128,
     its edges and its padding; hd 20 is the 16-bit generic kernel), ragged
     lengths around the 64-key tile, rows of MuNet's key matrix that start at
-    any alignment, one and two query groups per wave ((2, 130, 33) has 260
-    workgroups), and a key buffer whose last chunk ends at the allocation's
-    end.  Oracle: float64 attention with the reference's score roundings.
+    any alignment, and what lies past each operand's end (NaN) kept out of the
+    result.  Oracle: float64 attention with the reference's score roundings.
 
     Tolerances, against rows of max |ctx| about 1: fp32 2e-5, the scores' sum
     error (hd 2^-24 |q||k| scale, about 1e-6) plus T sums; 16-bit: 2^-8 (bf16)
@@ -193,6 +192,55 @@ def test_attention_head_sizes(hip, dt, hd, B, H, T, causal, textbook):
     ref = (torch.softmax(s, -1) @ vd).view(B, H, T, hd).permute(0, 2, 1, 3).reshape(B * T, H * hd)
     err = float((ctx.cpu().double() - ref).abs().max() / ref.abs().max())
     assert err <= (2e-5 if dt == F32 else 2e-2), err
+
+
+def _textbook_oracle(q, k, v, B, H, T, hd, causal, textbook):
+    """Attention in float64 with the reference's score roundings, of [B H T hd]
+    torch operands in their storage type, on MuNet's or textbook keys."""
+    import torch
+    tdt = q.dtype
+    qd, vd = (t.double().view(B * H, T, hd) for t in (q, v))
+    keys = k.double().view(B * H, T, hd).transpose(1, 2) if textbook else k.double().view(hd, B * H, T).permute(1, 0, 2)
+    scale = float(torch.tensor(1 / np.sqrt(hd), dtype=torch.float32).to(tdt))
+    s = qd @ keys.contiguous()
+    s = s * scale if tdt == torch.float32 else (s.to(tdt).double() * scale).to(tdt).double()
+    if causal:
+        s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=q.device).triu(1), -float("inf"))
+    return (torch.softmax(s, -1) @ vd).view(B, H, T, hd).permute(0, 2, 1, 3).reshape(B * T, H * hd)
+
+
+@pytest.mark.parametrize("dt", [F16, BF16])
+@pytest.mark.parametrize("hd", [72, 96, 104, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("textbook", [False, True])
+def test_attention_query_groups(hip, dt, hd, causal, textbook, monkeypatch):
+    """Two 16-row query groups per wave give the bits of one (each group's own
+    masks, running max and skipped tiles), at the edges of the 64- and 128-row
+    blocks, and both are within the rounding of float64: P and the result are
+    each rounded once, in units of max |ctx| 2^-8 (bf16) or 2^-10 (fp16, whose
+    half-ulp is 2^-11) times 2, and a score that the sum order moves by one
+    rounding moves its p by as much.  The automatic choice gives the same bits
+    on both sides of its border (512 wide workgroups, 1024 causal)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    tdt = {F16: torch.float16, BF16: torch.bfloat16}[dt]
+    attn = hip.attention_textbook if textbook else hip.attention
+    for B, H, T in ((1, 3, 1), (1, 3, 33), (2, 2, 64), (1, 3, 65), (2, 2, 127), (1, 3, 129), (1, 2, 200), (1, 1, 256), (4, 128, 130),
+                    (8, 127, 33), (8, 128, 33)):
+        q, k, v = (torch.randn(B * H * T * hd, device="cuda", generator=g).to(tdt) for _ in range(3))
+        outs = {}
+        for rw in ("1", "2", None):
+            if rw:
+                monkeypatch.setenv("MUNET_HIP_ATTN_RW", rw)
+            else:
+                monkeypatch.delenv("MUNET_HIP_ATTN_RW")
+            ctx = empty((B * T, H * hd), dt)
+            attn(q, k, v, ctx, B, H, T, hd, causal)
+            outs[rw] = ctx
+        assert torch.equal(outs["1"], outs["2"]) and torch.equal(outs["1"], outs[None]), (B, H, T)
+        ref = _textbook_oracle(q, k, v, B, H, T, hd, causal, textbook)
+        err = float((outs["2"].double() - ref).abs().max() / ref.abs().max())
+        assert err <= (2.0 ** -7 if dt == BF16 else 2.0 ** -9), (B, H, T, err)
 
 
 @pytest.mark.parametrize("dt", [F16, BF16])
