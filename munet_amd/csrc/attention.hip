@@ -169,7 +169,8 @@ __device__ __forceinline__ uint4 ld16_any(const uint16_t *p) {
 template <int DT, int HDP, int RW, bool TXT, bool P2>
 __global__ void __launch_bounds__(256, 2)
 flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-                     uint16_t *__restrict__ O, int B, int H, int T, int hd, int causal, float scale, float c2) {
+                     uint16_t *__restrict__ O, int B, int H, int T, int hd_, int causal, float scale, float c2) {
+  const int hd = P2 ? HD : hd_;  // (a constant: hd 64 lost 6 to 16% to the checks against it)
   constexpr int QB = 4 * 16 * RW;
   constexpr int KS = HDP / 32, ND = HDP / 16, NSUB = (HDP + 63) / 64;
   constexpr int NL = HDP / 32;   // 16-byte chunks each thread stages of a K or V tile
