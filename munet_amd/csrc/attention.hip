@@ -268,15 +268,17 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
 #pragma unroll
       for (int i = 0; i < NL; ++i) vr[i] = *reinterpret_cast<const uint4 *>(vp[i]);
     } else {
-      // ragged last tile: V (and textbook K) rows past T are zero; MuNet's K
-      // columns past T are masked after the product, so they may hold
-      // whatever follows, up to the buffer's last element
+      // ragged last tile: V rows past T are zero; keys past T are masked after
+      // the product, so textbook rows past T are ones (scores of zero would
+      // take the exact fp16 rounding: 300 x 8 heads of 96, 4 keys, 64 us against
+      // 41) and MuNet's columns hold whatever follows,
+      // up to the buffer's last element
 #pragma unroll
       for (int i = 0; i < NL; ++i) {
         const bool in = j0 + vrow[i] < T;
         vr[i] = in ? *reinterpret_cast<const uint4 *>(vp[i]) : make_uint4(0, 0, 0, 0);
         if constexpr (TXT) {
-          kr[i] = in ? *reinterpret_cast<const uint4 *>(kp[i]) : make_uint4(0, 0, 0, 0);
+          kr[i] = in ? *reinterpret_cast<const uint4 *>(kp[i]) : make_uint4(one2, one2, one2, one2);
         } else if (kend - kp[i] >= 8) {
           kr[i] = ld16_any(kp[i]);
         } else {
