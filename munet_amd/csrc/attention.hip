@@ -24,7 +24,8 @@
 //    tiles are copied to LDS in their natural layouts and the MFMA operands
 //    are read back transposed with ds_read_b64_tr_b16;
 //  * attention_f32 (attention_f32.hip; fp32, hd <= 128, hd % 4 == 0);
-//  * attn_generic_kernel (below): every other head size or alignment.
+//  * attn_generic_kernel (below): every other head size or alignment, and a few
+//    keys per head (launch_shapes.hpp).
 // The flash kernels compute S^T = K*Q^T and O^T = V^T*P^T so that every lane
 // owns one query row: P goes from the S accumulators into the PV operand
 // without touching LDS.  Scores are rounded like the reference
@@ -39,6 +40,7 @@
 
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
+#include "launch_shapes.hpp"
 
 namespace mh {
 
@@ -857,6 +859,7 @@ hipError_t attention(int dt, const void *q, const void *k, const void *v, void *
       hipLaunchKernelGGL((flash_attn_pipe_kernel<F16>), dim3(unsigned(items)), dim3(256), 0, st, Q, K, V, O, B, H, T, causal, c2, snake);
     return hipGetLastError();
   }
+  if (attention_by_rows(dt == F32, dt == F16, textbook, T, hd, long(B) * H)) force_generic = 1;
   if (!force_generic && (dt == BF16 || dt == F16) && aligned && hd % 8 == 0 && hd <= 128) {
     if (long((T + 63) / 64) * B * H > 0x7fffffffL) return hipErrorInvalidValue;
     return dt == BF16 ? flash_tr<BF16>(q, k, v, ctx, B, H, T, hd, causal, scale, textbook, st)

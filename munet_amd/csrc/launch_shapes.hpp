@@ -73,4 +73,20 @@ inline bool transpose_flat(long batch, long rows, long cols, int es, bool vec) {
   return n <= 1024 || batch > 65535 || (!vec && n * es <= 4096 + 7 * tiles);
 }
 
+// Whether attention over T keys in `blocks` (batch, head) blocks takes one wave
+// per query instead of the flash kernels, which do a whole 64-key tile for any
+// T and a few us for the smallest call.  Rows | tiles, us: fp32, 2400 blocks, hd
+// 8: T = 1 6.4 | 20.6, T = 8 15.8 | 20.2; hd 128: T = 1 17.9 | 62.6, T = 3 56.3 |
+// 64.4, T = 4 85.5 | 64.1 (textbook keys 71.6 | 82.4); 512 blocks, hd 128, T = 4
+// 18.1 | 15.3 (14.1 | 19.5); bf16, 2400 blocks, hd 96: T = 2 19.6 | 27.1, 16000
+// blocks of T = 3 187 | 166; fp16 187 | 259; 512 blocks, hd 96, T = 1 14.4 | 8.6.
+// (16-bit heads of 64 have always run on tiles; the rows' launch holds 65535
+// blocks.)
+inline bool attention_by_rows(bool f32, bool f16, bool textbook, int T, int hd, long blocks) {
+  if (blocks > 65535 || (!f32 && hd == 64)) return false;
+  if (long(T) * hd <= (f32 ? 64 : f16 ? 32 : 24)) return true;
+  if (f32) return textbook ? T <= 4 && blocks >= 256 : T <= (hd <= 96 ? 4 : 3) && blocks >= 1024;
+  return T <= (f16 && hd > 64 ? 4 : 2) && blocks >= 1024;
+}
+
 }  // namespace mh

@@ -73,6 +73,12 @@ int main() {
       {70000, 2, 1000, 4, true, true}};
   for (const auto &t : tr)
     if (mh::transpose_flat(t.b, t.r, t.c, t.es, t.vec) != t.flat) fail("transpose", t.b, t.r, t.c);
+  // a few keys of many heads by rows; long ones, and 16-bit heads of 64, by tiles
+  if (!mh::attention_by_rows(true, false, false, 1, 128, 2400) || !mh::attention_by_rows(true, false, true, 4, 64, 512) ||
+      !mh::attention_by_rows(false, true, false, 3, 96, 16000) || !mh::attention_by_rows(false, false, false, 3, 8, 2) ||
+      mh::attention_by_rows(false, false, false, 3, 96, 16000) || mh::attention_by_rows(false, false, false, 1, 64, 2400) ||
+      mh::attention_by_rows(true, false, false, 5, 64, 2400) || mh::attention_by_rows(true, false, false, 1, 8, 65536))
+    fail("attention", 0, 0, 0);
   for (long r : {1L, 67108863L, 4194303L, 4194304L, 16777216L, 67108864L, 2147483647L})
     for (int threads : {64, 256, 1024}) split(r, threads);
   std::printf("ok\n");

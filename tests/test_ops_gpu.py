@@ -209,6 +209,28 @@ def _textbook_oracle(q, k, v, B, H, T, hd, causal, textbook):
     return (torch.softmax(s, -1) @ vd).view(B, H, T, hd).permute(0, 2, 1, 3).reshape(B * T, H * hd)
 
 
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("textbook", [False, True])
+def test_attention_few_keys(hip, dt, causal, textbook):
+    """One to five keys in many and in few heads: both sides of the choice
+    between a wave per query and the flash kernels.  Tolerances as in
+    test_attention_query_groups; fp32 sums of hd products of scores about 1 and
+    of T terms, 2e-6."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(3)
+    tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dt]
+    for B, H in ((2, 3), (26, 10), (103, 10)):
+        for hd in (8, 24, 64, 96, 128):
+            for T in (1, 2, 3, 4, 5):
+                q, k, v = (torch.randn(B * H * T * hd, device="cuda", generator=g).to(tdt) for _ in range(3))
+                ctx = empty((B * T, H * hd), dt)
+                (hip.attention_textbook if textbook else hip.attention)(q, k, v, ctx, B, H, T, hd, causal)
+                ref = _textbook_oracle(q, k, v, B, H, T, hd, causal, textbook)
+                err = float((ctx.double() - ref).abs().max() / ref.abs().max())
+                assert err <= {F32: 2e-6, F16: 2.0 ** -9, BF16: 2.0 ** -7}[dt], (B, H, T, hd, err)
+
+
 @pytest.mark.parametrize("dt", [F16, BF16])
 @pytest.mark.parametrize("hd", [72, 96, 104, 128])
 @pytest.mark.parametrize("causal", [False, True])
