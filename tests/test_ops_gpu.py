@@ -231,6 +231,24 @@ def test_attention_few_keys(hip, dt, causal, textbook):
                 assert err <= {F32: 2e-6, F16: 2.0 ** -9, BF16: 2.0 ** -7}[dt], (B, H, T, hd, err)
 
 
+@pytest.mark.parametrize("dt,bound", [(F16, 2.74e-4), (BF16, 2.21e-3)])
+@pytest.mark.parametrize("T", [237, 250])
+def test_attention_ragged_length_error(hip, dt, bound, T):
+    """Heads of 64 on lengths off a multiple of 8 subtract the exact running
+    max, so that a row's largest p carries no rounding: the relative 2-norm
+    error for scores about 1 is 2.68e-4 / 2.17e-3, against 2.81e-4 / 2.26e-3
+    with the max raised in steps of 2^8."""
+    import torch
+    B, H, hd = 8, 8, 64
+    g = torch.Generator(device="cuda").manual_seed(T)
+    tdt = {F16: torch.float16, BF16: torch.bfloat16}[dt]
+    q, k, v = (torch.randn(B * H * T * hd, device="cuda", generator=g).to(tdt) for _ in range(3))
+    ctx = empty((B * T, H * hd), dt)
+    hip.attention(q, k, v, ctx, B, H, T, hd, False)
+    ref = _textbook_oracle(q, k, v, B, H, T, hd, False, False)
+    assert float((ctx.double() - ref).norm() / ref.norm()) <= bound
+
+
 @pytest.mark.parametrize("dt", [F16, BF16])
 @pytest.mark.parametrize("hd", [72, 96, 104, 128])
 @pytest.mark.parametrize("causal", [False, True])
