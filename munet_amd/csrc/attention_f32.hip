@@ -28,10 +28,18 @@
 // are single-buffered in LDS with the next tile in registers: 32 KB at hd 64
 // leaves room for several workgroups per CU.  Encoder layer of 8 x 250 tokens,
 // 8 heads of 64: the block took 382 us with the one-wave-per-query kernel that
-// this replaces, 215 us with this one, at the same error against float64.
+// this replaces, 215 us with this one (the other kernels as they were).
 //
 // Precision: exp(v - m) with m the exact running row max, its base-2 argument
-// carried in two floats (the one-float product loses |v - m| 2^-24).
+// carried in two floats (the one-float product loses |v - m| 2^-24); row sums in
+// doubles, scores and outputs each in two accumulators (even and odd elements
+// d, even and odd keys), which halves the variance of a long sum, and one rounding of
+// their double sum over the row sum.  Against float64 that is 0.66 to 0.88 of
+// the error of the one-wave-per-query kernel, whose exponentials, sum and
+// division are doubles, over 2 to 4000 keys, heads of 8 to 128 and scores of 0.25
+// to 9; with one accumulator each and fp32 row sums it had been 1.00 to 1.26
+// of it.  Time: up to 6% more than that form (8 x 250 keys, 8 heads of 64 19.5
+// -> 20.2 us).
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
 
@@ -55,7 +63,7 @@ __device__ __forceinline__ float exp_neg(float x) {
 }
 
 template <int NG, int CW, bool TXT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, NG * CW == 4 && !TXT ? 3 : NG * CW == 8 ? 2 : 1)
 flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
                       float *__restrict__ O, int B, int H, int T, int hd, int causal, float scale) {
   constexpr int HDP = NG * 16 * CW, KS = HDP / 16, VC = HDP / 4;  // VC: 16-byte chunks of a V row
@@ -80,19 +88,27 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
     qf[ks] = d < hd ? *reinterpret_cast<const f32x4 *>(Q + (long(bh) * T + min(i, T - 1)) * hd + d)
                     : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  f32x4 o[NG][CW];
+  f32x4 o[2][NG][CW];
 #pragma unroll
-  for (int g = 0; g < NG; ++g)
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int w = 0; w < CW; ++w) o[g][w] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -3.4028234e38f, l = 0.f;
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int w = 0; w < CW; ++w) o[h][g][w] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -3.4028234e38f;
+  double l = 0.0;
 
-  // staging: chunk id = tid + 256 n of a tile
-  const float *kp[NL], *vp[NL];
-  int kst[NL], vst[NL], vrow[NL];
-  bool kin[NL], vin[NL];
+  // staging: chunk id = tid + 256 n of a tile.  Where 256 chunks are whole rows
+  // (kEven) the n-th chunk lies a fixed distance from the first, and so do the
+  // rows of MuNet's keys: one pointer for all (an array of them cost 50
+  // registers and hd 128 its second wave per SIMD).
+  constexpr bool kEven = 256 % VC == 0;
+  constexpr int NP = kEven ? 1 : NL, RS = 256 / VC;
+  const float *kp[TXT ? NP : 1], *vp[NP];
+  int kst[TXT ? NP : 1], vst[NP], vrow[NP];
+  bool vin[NP];  // (textbook keys: in the same way)
 #pragma unroll
-  for (int n = 0; n < NL; ++n) {
+  for (int n = 0; n < NP; ++n) {
     const int id = tid + 256 * n, row = id / VC, c = id % VC;
     vrow[n] = row;
     vin[n] = 4 * c < hd;
@@ -100,51 +116,64 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
     vp[n] = Vb + voff;
     vst[n] = row * HDP + 4 * c;
     if constexpr (TXT) {
-      kin[n] = vin[n];
       kp[n] = Kb + voff;
       kst[n] = row * HDP + 4 * (c ^ (row & 7));
-    } else {
-      const int d = id >> 4;
-      kin[n] = d < hd;
-      kp[n] = Kb + long(min(d, hd - 1)) * N + 4 * (id & 15);
-      kst[n] = d * KB + 4 * (id & 15);
     }
-    if (!kin[n]) *reinterpret_cast<f32x4 *>(ks_ + kst[n]) = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  const int kd = tid >> 4;  // MuNet's keys: row kd + 16 n of the tile
+  if constexpr (!TXT) {
+    kp[0] = Kb + kd * N + 4 * (tid & 15);
+    kst[0] = kd * KB + 4 * (tid & 15);
+  }
+  // index and row distance of the n-th chunk
+  auto pi = [](int n) { return kEven ? 0 : n; };
+  auto rs = [](int n) { return kEven ? n * RS : 0; };
+  auto kin = [&](int n) { return TXT ? vin[pi(n)] : kd + 16 * n < hd; };
+  auto kptr = [&](int n) { return TXT ? kp[pi(n)] + long(rs(n)) * hd : kp[0] + 16 * n * N; };
+  auto vptr = [&](int n) { return vp[pi(n)] + long(rs(n)) * hd; };
+  auto kdst = [&](int n) { return ks_ + (TXT ? kst[pi(n)] + rs(n) * HDP : kst[0] + 16 * n * KB); };
+  auto vdst = [&](int n) { return vs_ + vst[pi(n)] + rs(n) * HDP; };
+#pragma unroll
+  for (int n = 0; n < NL; ++n)
+    if (!kin(n)) *reinterpret_cast<f32x4 *>(kdst(n)) = f32x4{0.f, 0.f, 0.f, 0.f};
   const long kstep = TXT ? long(KB) * hd : KB, vstep = long(KB) * hd;
   f32x4 kr[NL], vr[NL];
   auto gload = [&](int j0) {
     if (j0 + KB <= T) {
 #pragma unroll
       for (int n = 0; n < NL; ++n) {
-        if constexpr (TXT) kr[n] = *reinterpret_cast<const f32x4 *>(kp[n]);
-        else kr[n] = *reinterpret_cast<const f32x4_any *>(kp[n]);
-        vr[n] = *reinterpret_cast<const f32x4 *>(vp[n]);
+        if constexpr (TXT) kr[n] = *reinterpret_cast<const f32x4 *>(kptr(n));
+        else if (kin(n)) kr[n] = *reinterpret_cast<const f32x4_any *>(kptr(n));
+        vr[n] = *reinterpret_cast<const f32x4 *>(vptr(n));
       }
     } else {
 #pragma unroll
       for (int n = 0; n < NL; ++n) {
-        const bool in = j0 + vrow[n] < T;
-        const f32x4 vv = *reinterpret_cast<const f32x4 *>(in ? vp[n] : Vb);
+        const bool in = j0 + vrow[pi(n)] + rs(n) < T;
+        const f32x4 vv = *reinterpret_cast<const f32x4 *>(in ? vptr(n) : Vb);
 #pragma unroll
         for (int e = 0; e < 4; ++e) vr[n][e] = in ? vv[e] : 0.f;
         if constexpr (TXT) {
-          const f32x4 kv = *reinterpret_cast<const f32x4 *>(in ? kp[n] : Kb);
+          const f32x4 kv = *reinterpret_cast<const f32x4 *>(in ? kptr(n) : Kb);
 #pragma unroll
           for (int e = 0; e < 4; ++e) kr[n][e] = in ? kv[e] : 0.f;
-        } else if (kend - kp[n] >= 4) {
-          kr[n] = *reinterpret_cast<const f32x4_any *>(kp[n]);
-        } else {
+        } else if (kin(n)) {
+          const long left = kend - kptr(n);
+          if (left >= 4) {
+            kr[n] = *reinterpret_cast<const f32x4_any *>(kptr(n));
+          } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) kr[n][e] = kend - kp[n] > e ? kp[n][e] : 0.f;
+            for (int e = 0; e < 4; ++e) kr[n][e] = left > e ? kptr(n)[e] : 0.f;
+          }
         }
       }
     }
 #pragma unroll
-    for (int n = 0; n < NL; ++n) {
-      kp[n] += kstep;
+    for (int n = 0; n < NP; ++n) {
+      if constexpr (TXT) kp[n] += kstep;
       vp[n] += vstep;
     }
+    if constexpr (!TXT) kp[0] += kstep;
   };
 
   const int kv_end = causal ? min(T, q0 + KB) : T;
@@ -155,15 +184,15 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
     __syncthreads();  // the previous tile has been read
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
-      if (kin[n]) *reinterpret_cast<f32x4 *>(ks_ + kst[n]) = kr[n];
-      if (vin[n]) *reinterpret_cast<f32x4 *>(vs_ + vst[n]) = vr[n];
+      if (kin(n)) *reinterpret_cast<f32x4 *>(kdst(n)) = kr[n];
+      if (vin[pi(n)]) *reinterpret_cast<f32x4 *>(vdst(n)) = vr[n];
     }
     __syncthreads();
     if (t + 1 < ntiles) gload(j0 + KB);
 
-    f32x4 s[4];
+    f32x4 s[4], s1[4];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) s[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < 4; ++x) s[x] = s1[x] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (TXT) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -174,7 +203,10 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int x = 0; x < 4; ++x) s[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[x][e], qf[ks][e], s[x], 0, 0, 0);
+          for (int x = 0; x < 4; ++x) {
+            f32x4 &c = (e & 1 ? s1 : s)[x];
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[x][e], qf[ks][e], c, 0, 0, 0);
+          }
       }
     } else {
 #pragma unroll
@@ -183,7 +215,10 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
         for (int e = 0; e < 4; ++e) {
           const f32x4 kf = *reinterpret_cast<const f32x4 *>(ks_ + (16 * ks + 4 * lg + e) * KB + 4 * li);
 #pragma unroll
-          for (int x = 0; x < 4; ++x) s[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[x], qf[ks][e], s[x], 0, 0, 0);
+          for (int x = 0; x < 4; ++x) {
+            f32x4 &c = (e & 1 ? s1 : s)[x];
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[x], qf[ks][e], c, 0, 0, 0);
+          }
         }
     }
 
@@ -194,7 +229,7 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
     for (int x = 0; x < 4; ++x)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float v = __fmul_rn(s[x][e], scale);
+        float v = __fmul_rn(__fadd_rn(s[x][e], s1[x][e]), scale);
         if (edge && (TXT ? 16 * x + 4 * lg + e : 16 * lg + 4 * e + x) > lim) v = -INFINITY;
         s[x][e] = v;
         mx = fmaxf(mx, v);
@@ -205,16 +240,18 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
       m = mnew;
       l *= alpha;
 #pragma unroll
-      for (int g = 0; g < NG; ++g)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int w = 0; w < CW; ++w) o[g][w] *= alpha;
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int w = 0; w < CW; ++w) o[h][g][w] *= alpha;
     }
 #pragma unroll
     for (int x = 0; x < 4; ++x)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         s[x][e] = exp_neg(s[x][e] - m);
-        l += s[x][e];
+        l += double(s[x][e]);
       }
 #pragma unroll
     for (int x = 0; x < 4; ++x)
@@ -225,13 +262,18 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
         for (int g = 0; g < NG; ++g) {
           const vcw vf = *reinterpret_cast<const vcw *>(vs_ + row * HDP + CW * (16 * g + li));
 #pragma unroll
-          for (int w = 0; w < CW; ++w) o[g][w] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[w], s[x][e], o[g][w], 0, 0, 0);
+          for (int w = 0; w < CW; ++w) {
+            f32x4 &c = o[(TXT ? e : x) & 1][g][w];  // neighbouring keys apart
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[w], s[x][e], c, 0, 0, 0);
+          }
         }
       }
   }
 
-  l = xor32_add(xor16_add(l));
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
   if (i >= T) return;
+  const double inv = 1.0 / l;
   const int b = bh / H, h = bh - b * H;
   float *dst = O + (long(b) * T + i) * (long(H) * hd) + long(h) * hd;
 #pragma unroll
@@ -242,7 +284,7 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
       if (d >= hd) continue;
       vcw w4;
 #pragma unroll
-      for (int w = 0; w < CW; ++w) w4[w] = o[g][w][e] / l;
+      for (int w = 0; w < CW; ++w) w4[w] = float((double(o[0][g][w][e]) + double(o[1][g][w][e])) * inv);
       *reinterpret_cast<vcw *>(dst + d) = w4;
     }
 }
