@@ -164,6 +164,32 @@ __device__ __forceinline__ uint4 ld16_any(const uint16_t *p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// One causal row again, over keys 0..qi alone, by one wave: lane j of a group of
+// 64 keys takes key j's score and p (against the row's final max m and 1 / sum
+// of the flash kernel), then lanes d and d + 64 the output columns.
+template <int DT, bool TXT>
+__device__ __forceinline__ void causal_row(const uint16_t *q, const uint16_t *Kb, const uint16_t *Vb, uint16_t *dst, int qi,
+                                        int hd, long N, float scale, float c2, float m, float inv) {
+  typedef Store<DT> S;
+  const int lane = threadIdx.x & 63;
+  float a0 = 0.f, a1 = 0.f;
+  for (int j0 = 0; j0 <= qi; j0 += 64) {
+    const int j = min(j0 + lane, qi);
+    float acc = 0.f;
+    for (int d = 0; d < hd; ++d) acc += S::dec(q[d]) * S::dec(TXT ? Kb[long(j) * hd + d] : Kb[d * N + j]);
+    const float v = S::round(S::round(acc) * scale);
+    const float p = S::dec(AttnMfma<DT>::cvt(__builtin_amdgcn_exp2f(__builtin_fmaf(v, c2, -m))));
+    for (int k = 0; k < 64 && j0 + k <= qi; ++k) {
+      const float pk = __shfl(p, k, 64);
+      const uint16_t *vr = Vb + long(j0 + k) * hd;
+      if (lane < hd) a0 += pk * S::dec(vr[lane]);
+      if (lane + 64 < hd) a1 += pk * S::dec(vr[lane + 64]);
+    }
+  }
+  if (lane < hd) dst[lane] = S::enc(a0 * inv);
+  if (lane + 64 < hd) dst[lane + 64] = S::enc(a1 * inv);
+}
+
 // TXT (textbook keys): K is head-split like V, key j of block bh at row
 // bh*T + j; its tile is staged in natural [j][d] layout (the swz pattern, 64
 // columns per sub-tile) and the MFMA's K operand is read straight, without
@@ -434,9 +460,33 @@ flash_attn_tr_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict_
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
     const int i = wrow0 + r * 16 + li;
-    if (i >= T) continue;
     const float inv = 1.0f / osum[r][0];
     uint16_t *dst = O + (long(b) * T + i) * E + long(h) * hd;
+    // An infinity or NaN in a masked row of V reaches the queries before it in
+    // its tile as 0 * inf: a row with a NaN that its scores do not account for
+    // is summed again over its own keys.  (Heads of 64 keep MuNet's own
+    // behaviour, whose dense product spreads such a value to every row.)
+    bool redo = false;
+    if constexpr (!P2) {
+      if (causal) {
+        bool nan = false;
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+          if (dt * 16 + lg * 4 < hd)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) nan |= o[r][dt][e] != o[r][dt][e];
+        uint64_t rows = __ballot(nan && i < T && osum[r][0] == osum[r][0]);
+        rows |= rows >> 32;
+        rows = (rows | rows >> 16) & 0xffff;
+        redo = rows >> li & 1;
+        for (; rows; rows &= rows - 1) {
+          const int row = __builtin_ctzll(rows), qi = wrow0 + r * 16 + row;
+          causal_row<DT, TXT>(Q + (long(bh) * T + qi) * hd, Kb, Vb, O + (long(b) * T + qi) * E + long(h) * hd, qi, hd, N,
+                              scale, c2, __shfl(mrow[r], row, 64), __shfl(inv, row, 64));
+        }
+      }
+    }
+    if (i >= T || redo) continue;
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt) {
       if (dt * 16 + lg * 4 >= hd) continue;

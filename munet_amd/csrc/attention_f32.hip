@@ -62,8 +62,32 @@ __device__ __forceinline__ float exp_neg(float x) {
   return __fmaf_rn(p, __fmul_rn(lo, kLn2), p);
 }
 
+// One causal row again, over keys 0..qi alone, by one wave (see the end of the
+// kernel): lane j of a group of 64 keys takes key j's p against the row's max m,
+// then lanes d and d + 64 the output columns.
+template <bool TXT>
+__device__ __forceinline__ void causal_row(const float *q, const float *Kb, const float *Vb, float *dst, int qi, int hd,
+                                           long N, float scale, float m, double inv) {
+  const int lane = threadIdx.x & 63;
+  float a0 = 0.f, a1 = 0.f;
+  for (int j0 = 0; j0 <= qi; j0 += 64) {
+    const int j = min(j0 + lane, qi);
+    float acc = 0.f;
+    for (int d = 0; d < hd; ++d) acc = __fmaf_rn(q[d], TXT ? Kb[long(j) * hd + d] : Kb[d * N + j], acc);
+    const float p = exp_neg(__fmul_rn(acc, scale) - m);
+    for (int k = 0; k < 64 && j0 + k <= qi; ++k) {
+      const float pk = __shfl(p, k, 64);
+      const float *vr = Vb + long(j0 + k) * hd;
+      if (lane < hd) a0 = __fmaf_rn(pk, vr[lane], a0);
+      if (lane + 64 < hd) a1 = __fmaf_rn(pk, vr[lane + 64], a1);
+    }
+  }
+  if (lane < hd) dst[lane] = float(double(a0) * inv);
+  if (lane + 64 < hd) dst[lane + 64] = float(double(a1) * inv);
+}
+
 template <int NG, int CW, bool TXT>
-__global__ void __launch_bounds__(256, NG * CW == 4 && !TXT ? 3 : NG * CW == 8 ? 2 : 1)
+__global__ void __launch_bounds__(256, NG * CW == 2 ? (TXT ? 3 : 4) : NG * CW == 4 ? (TXT ? 2 : 3) : 2)
 flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
                       float *__restrict__ O, int B, int H, int T, int hd, int causal, float scale) {
   constexpr int HDP = NG * 16 * CW, KS = HDP / 16, VC = HDP / 4;  // VC: 16-byte chunks of a V row
@@ -272,10 +296,37 @@ flash_attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, 
 
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  if (i >= T) return;
   const double inv = 1.0 / l;
   const int b = bh / H, h = bh - b * H;
-  float *dst = O + (long(b) * T + i) * (long(H) * hd) + long(h) * hd;
+  float *const out = O + long(b) * T * (long(H) * hd) + long(h) * hd;
+  // An infinity or NaN in a masked row of V reaches the queries before it in
+  // its tile as 0 * inf: a row with a NaN that its scores do not account for is
+  // summed again over its own keys.
+  if (causal) {
+    bool nan = false;
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (CW * (16 * g + 4 * lg + e) < hd)
+#pragma unroll
+          for (int w = 0; w < CW; ++w) {
+            const float v = o[0][g][w][e] + o[1][g][w][e];
+            nan |= v != v;
+          }
+    uint64_t rows = __ballot(nan && i < T && l == l);
+    rows |= rows >> 32;
+    rows = (rows | rows >> 16) & 0xffff;
+    const bool redo = rows >> li & 1;
+    for (; rows; rows &= rows - 1) {
+      const int row = __builtin_ctzll(rows), qi = wrow0 + row;
+      causal_row<TXT>(Q + (long(bh) * T + qi) * hd, Kb, Vb, out + qi * (long(H) * hd), qi, hd, N, scale,
+                      __shfl(m, row, 64), __shfl(inv, row, 64));
+    }
+    if (redo) return;
+  }
+  if (i >= T) return;
+  float *dst = out + i * (long(H) * hd);
 #pragma unroll
   for (int g = 0; g < NG; ++g)
 #pragma unroll

@@ -231,6 +231,38 @@ def test_attention_few_keys(hip, dt, causal, textbook):
                 assert err <= {F32: 2e-6, F16: 2.0 ** -9, BF16: 2.0 ** -7}[dt], (B, H, T, hd, err)
 
 
+@pytest.mark.parametrize("dt,hd,rw", [(F16, 32, "1"), (BF16, 40, "1"), (BF16, 96, "1"), (BF16, 96, "2"), (F16, 128, "1"),
+                                      (F16, 128, "2"), (F32, 16, "1"), (F32, 64, "1"), (F32, 96, "1"), (F32, 128, "1")])
+@pytest.mark.parametrize("textbook", [False, True])
+def test_causal_rows_ignore_later_values(hip, dt, hd, rw, textbook, monkeypatch):
+    """An infinity or a NaN in row j of V reaches the queries from j on and no
+    query before it, in its own 64-key tile (where the flash kernels multiply
+    it by a zero probability) or in an earlier one; every other value is that
+    of the finite V.  A NaN in Q makes its own row NaN and no other."""
+    import torch
+    monkeypatch.setenv("MUNET_HIP_ATTN_RW", rw)
+    tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dt]
+    B, H, T = 2, 3, 165
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    q, k, v = (torch.randn(B * H * T * hd, device="cuda", generator=g).to(tdt) for _ in range(3))
+    ref = _textbook_oracle(q, k, v, B, H, T, hd, True, textbook).view(B, T, H, hd)
+    bad = torch.zeros(B, T, H, hd, dtype=torch.bool, device="cuda")
+    vv, qq = v.view(B, H, T, hd), q.view(B, H, T, hd)
+    for b, h, j, d, x in ((0, 0, 40, 3, float("inf")), (0, 0, 164, 5, float("nan")), (0, 2, 63, hd - 1, -float("inf")),
+                          (1, 1, 100, 0, float("nan")), (1, 1, 150, 7, float("inf"))):
+        vv[b, h, j, d] = x
+        bad[b, j:, h, d] = True
+    qq[1, 0, 70, 2] = float("nan")
+    bad[1, 70, 0] = True
+    ctx = empty((B * T, H * hd), dt)
+    (hip.attention_textbook if textbook else hip.attention)(q, k, v, ctx, B, H, T, hd, True)
+    y = ctx.double().view(B, T, H, hd)
+    assert torch.equal(~torch.isfinite(y), bad)
+    assert bool((y[0, 40:, 0, 3] == float("inf")).all()) and bool((y[0, 63:, 2, hd - 1] == -float("inf")).all())
+    err = float((y - ref)[~bad].abs().max() / ref.abs().max())
+    assert err <= {F32: 2e-6, F16: 2.0 ** -9, BF16: 2.0 ** -7}[dt], err
+
+
 @pytest.mark.parametrize("hd", [16, 64, 96, 128])
 @pytest.mark.parametrize("textbook", [False, True])
 def test_f32_attention_error_not_above_rows(hip, hd, textbook):
