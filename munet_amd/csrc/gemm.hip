@@ -278,14 +278,15 @@ hipError_t launch_cfg(const void *A, const void *Bt, int M, int N, int K, long l
   else vec = vec && (lda % E == 0) && (sa % E == 0);
   dim3 grid(tiles, 1, batch);
   const ConvArgs none{};
-  // Instantiated variants, 16-bit: the aligned (VEC) path for every tile; the
+  // Instantiated variants: the aligned (VEC) path for every tile; the
   // unaligned path only for the 64x64 tile (host falls back to it); the conv
-  // loader for tiles up to 256x128.
+  // loader for tiles up to 256x128.  fp32: the 64x64 tile alone.
   constexpr bool kSmall = (BM == 64 && BN == 64);
   if constexpr (DT == F32) {
-    // whole 16-byte chunks run on gemm_f32.hip
-    if constexpr (!kSmall) return hipErrorInvalidValue;
+    static_assert(kSmall, "fp32 runs on 64x64 tiles");
+    if (cv && vec) launch_one<DT, BM, BN, WGM, WGN, true, true>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, *cv);
     else if (cv) launch_one<DT, BM, BN, WGM, WGN, false, true>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, *cv);
+    else if (vec) launch_one<DT, BM, BN, WGM, WGN, true, false>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, none);
     else launch_one<DT, BM, BN, WGM, WGN, false, false>(grid, lds, st, A, Bt, M, N, K, lda, ldb, sa, sb, sc, ep, none);
   } else if (cv) {
     if constexpr (BM * BN <= 256 * 128 && WGM * WGN == 4) {
@@ -303,61 +304,53 @@ hipError_t launch_cfg(const void *A, const void *Bt, int M, int N, int K, long l
   return hipGetLastError();
 }
 
-// Choose the block tile that minimises (waves of tiles) x (tile cost) on 256
+// 16 bits: the block tile that minimises (waves of tiles) x (tile cost) on 256
 // CUs, preferring larger tiles for operand reuse when the wave count ties.
+// fp32 (what gemm_f32.hip does not take: unaligned operands, 2 GiB and more
+// under a tile's rows): 64x64.
 template <int DT>
 hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long lda, long ldb, int batch, long sa,
                      long sb, long sc, const EpiArgs &ep, const ConvArgs *cv, int tile_hint, hipStream_t st) {
-  struct Cand { int bm, bn; double cost; };
-  const int kCU = 256;
-  Cand cands[5] = {{256, 256, 4.0}, {256, 128, 2.0}, {128, 128, 1.0}, {128, 64, 0.55}, {64, 64, 0.3}};
-  int best = 2;
-  if (tile_hint >= 0 && tile_hint < 8) {
-    best = tile_hint;
-  } else if (DT != F32 && !cv && long((M + 255) / 256) * ((N + 255) / 256) * batch >= 1024) {
-    best = 7;  // 256x256, 8 waves: measured best for large GEMMs (LM head)
-  } else if (DT != F32 && !cv && long((M + 127) / 128) * ((N + 127) / 128) * batch >= 128) {
-    best = 2;  // 128x128, two blocks per CU: measured best for the layer GEMMs
+  if constexpr (DT == F32) {
+    return launch_cfg<DT, 64, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
   } else {
-    double best_t = 1e30;
-    for (int c = 0; c < 5; ++c) {
-      const long tiles = long((M + cands[c].bm - 1) / cands[c].bm) * ((N + cands[c].bn - 1) / cands[c].bn) * batch;
-      const long waves = (tiles + kCU - 1) / kCU;
-      // per-tile cost grows with the tile area, discounted for better reuse
-      const double t = double(waves) * cands[c].cost;
-      if (t < best_t * 0.999) { best_t = t; best = c; }
+    struct Cand { int bm, bn; double cost; };
+    const int kCU = 256;
+    Cand cands[5] = {{256, 256, 4.0}, {256, 128, 2.0}, {128, 128, 1.0}, {128, 64, 0.55}, {64, 64, 0.3}};
+    int best = 2;
+    if (tile_hint >= 0 && tile_hint < 8) {
+      best = tile_hint;
+    } else if (!cv && long((M + 255) / 256) * ((N + 255) / 256) * batch >= 1024) {
+      best = 7;  // 256x256, 8 waves: measured best for large GEMMs (LM head)
+    } else if (!cv && long((M + 127) / 128) * ((N + 127) / 128) * batch >= 128) {
+      best = 2;  // 128x128, two blocks per CU: measured best for the layer GEMMs
+    } else {
+      double best_t = 1e30;
+      for (int c = 0; c < 5; ++c) {
+        const long tiles = long((M + cands[c].bm - 1) / cands[c].bm) * ((N + cands[c].bn - 1) / cands[c].bn) * batch;
+        const long waves = (tiles + kCU - 1) / kCU;
+        // per-tile cost grows with the tile area, discounted for better reuse
+        const double t = double(waves) * cands[c].cost;
+        if (t < best_t * 0.999) { best_t = t; best = c; }
+      }
     }
-  }
-  constexpr int E = Mfma<DT>::kElems;
-  bool vec = (ldb % E == 0) && (sb % E == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)Bt % 16 == 0);
-  if (cv) vec = vec && (cv->iC % E == 0) && (cv->ldx % E == 0);
-  else vec = vec && (lda % E == 0) && (sa % E == 0);
-  if (!vec || DT == F32) best = 4;
-  if (cv && best == 0) best = 1;  // 256x256 only for plain GEMMs
-  if (cv && best >= 5) best = 2;  // 8-wave tiles only for plain GEMMs
-  switch (best) {
-  case 0:
-    if constexpr (DT != F32) return launch_cfg<DT, 256, 256, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  case 1:
-    if constexpr (DT != F32) return launch_cfg<DT, 256, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  case 2:
-    if constexpr (DT != F32) return launch_cfg<DT, 128, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  case 3:
-    if constexpr (DT != F32) return launch_cfg<DT, 128, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  case 5:
-    if constexpr (DT != F32) return launch_cfg<DT, 256, 128, 4, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  case 6:
-    if constexpr (DT != F32) return launch_cfg<DT, 128, 256, 2, 4>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  case 7:
-    if constexpr (DT != F32) return launch_cfg<DT, 256, 256, 4, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
-    return hipErrorInvalidValue;
-  default: return launch_cfg<DT, 64, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    constexpr int E = Mfma<DT>::kElems;
+    bool vec = (ldb % E == 0) && (sb % E == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)Bt % 16 == 0);
+    if (cv) vec = vec && (cv->iC % E == 0) && (cv->ldx % E == 0);
+    else vec = vec && (lda % E == 0) && (sa % E == 0);
+    if (!vec) best = 4;
+    if (cv && best == 0) best = 1;  // 256x256 only for plain GEMMs
+    if (cv && best >= 5) best = 2;  // 8-wave tiles only for plain GEMMs
+    switch (best) {
+    case 0: return launch_cfg<DT, 256, 256, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    case 1: return launch_cfg<DT, 256, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    case 2: return launch_cfg<DT, 128, 128, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    case 3: return launch_cfg<DT, 128, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    case 5: return launch_cfg<DT, 256, 128, 4, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    case 6: return launch_cfg<DT, 128, 256, 2, 4>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    case 7: return launch_cfg<DT, 256, 256, 4, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    default: return launch_cfg<DT, 64, 64, 2, 2>(A, Bt, M, N, K, lda, ldb, batch, sa, sb, sc, ep, cv, st);
+    }
   }
 }
 
@@ -368,9 +361,10 @@ hipError_t gemm_nt(int dt, const void *A, const void *Bt, int M, int N, int K, l
   if (M <= 0 || N <= 0 || batch <= 0) return hipSuccess;
   if (tile_hint < 0) {
     // MUNET_HIP_GEMM_TILE forces a kernel and block tile for tests and tuning:
-    // 0-6 direct-to-LDS kernel, 100-107 general kernel, 200-203, 207-212,
-    // 216, 217 and 219-227 pipelined kernel, 300-302 fp32 kernel.  Read at every call so a process can
-    // switch it between calls; any other code is an error.
+    // 0-6 direct-to-LDS kernel, 100-107 general kernel (fp32: its one tile),
+    // 200-203, 207-212, 216, 217 and 219-227 pipelined kernel, 300-302 fp32
+    // kernel.  Read at every call so a process can switch it between calls; any
+    // other code is an error.
     const char *force = std::getenv("MUNET_HIP_GEMM_TILE");
     if (force && *force) {
       tile_hint = std::atoi(force);
@@ -544,7 +538,9 @@ hipError_t conv_nhwc(int dt, const void *x, const void *w_ohwi, const ConvArgs &
   const int M = cv.B * cv.oH * cv.oW, K = cv.kH * cv.kW * cv.iC;
   if (M <= 0 || oC <= 0) return hipSuccess;
   // 16-bit convolutions with whole 64-channel slabs run on the pipelined
-  // kernel; MUNET_HIP_CONV_KERNEL=general (read per call) keeps this one
+  // kernel, fp32 ones of whole 16-byte chunks on gemm_f32.hip (MUNET_HIP_CONV_TILE
+  // = 300, 301 or 302 names its tile); MUNET_HIP_CONV_KERNEL=general keeps this
+  // one (both read per call)
   const char *ck = std::getenv("MUNET_HIP_CONV_KERNEL");
   const bool general = ck && std::string(ck) == "general";
   if (tile_hint < 0 && !general && (dt == F16 || dt == BF16) && cv.kH == 1 && cv.kW == 1 && cv.s == 1 && cv.p == 0 &&
@@ -557,8 +553,11 @@ hipError_t conv_nhwc(int dt, const void *x, const void *w_ohwi, const ConvArgs &
     return gemm_pipe_conv(dt, x, w_ohwi, cv, oC, ep, st);
   switch (dt) {
   case F32:
-    if (tile_hint < 0 && gemm_f32_ok(x, w_ohwi, K, 0, K, 0, 0, &cv))
-      return gemm_f32((const float *)x, (const float *)w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, -1, st);
+    if (tile_hint < 0 && !general && gemm_f32_ok(x, w_ohwi, K, 0, K, 0, 0, &cv)) {
+      const char *ct = std::getenv("MUNET_HIP_CONV_TILE");
+      return gemm_f32((const float *)x, (const float *)w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv,
+                      ct ? std::atoi(ct) - 300 : -1, st);
+    }
     return launch_dt<F32>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);
   case F16: return launch_dt<F16>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);
   case BF16: return launch_dt<BF16>(x, w_ohwi, M, oC, K, 0, K, 1, 0, 0, 0, ep, &cv, tile_hint, st);

@@ -1,8 +1,9 @@
 // fp32 MFMA GEMM and implicit-GEMM convolution for gfx950: C[M,N] = A[M,K] *
 // Bt[N,K]^T with the fused epilogue of gemm_common.hpp, full fp32 products
 // and sums (v_mfma_f32_16x16x4f32).  Operands in whole 16-byte chunks (K, the
-// row strides and a convolution's channels multiples of 4, 16-byte aligned);
-// every other fp32 product runs on gemm.hip's general kernel.
+// row strides and a convolution's channels multiples of 4, 16-byte aligned)
+// with less than 2 GiB under a tile's rows; every other fp32 product runs on
+// gemm.hip's general kernel.
 //
 // Bound: the fp32 matrix rate, 1/16 of the bf16 one (157 TFLOP/s nominal; a
 // register-only loop of this instruction reaches 154, a large library product
@@ -35,6 +36,7 @@
 #include "mh_common.hpp"
 #include "mh_kernels.hpp"
 #include "gemm_common.hpp"
+#include "launch_shapes.hpp"
 
 namespace mh {
 namespace {
@@ -93,7 +95,8 @@ gemm_f32_kernel(const float *__restrict__ A, const float *__restrict__ Bt, int M
   long abase, alen;
   if constexpr (CONV) {
     const int img = cv.oH * cv.oW, b0 = m0 / img;
-    abase = long(b0) * cv.iH * cv.iW * cv.ldx;
+    const int row0 = conv_base_row((m0 - b0 * img) / cv.oW, cv.iH, cv.s, cv.p);
+    abase = (long(b0) * cv.iH + row0) * cv.iW * cv.ldx;
     alen = long(cv.B) * cv.iH * cv.iW * cv.ldx - (cv.ldx - cv.iC) - abase;
 #pragma unroll
     for (int i = 0; i < ACH; ++i) {
@@ -101,8 +104,9 @@ gemm_f32_kernel(const float *__restrict__ A, const float *__restrict__ Bt, int M
       const int ow = m % cv.oW, t = m / cv.oW, oh = t % cv.oH, b = t / cv.oH;
       ih0[i] = oh * cv.s - cv.p;
       iw0[i] = ow * cv.s - cv.p;
-      // element offset of tap (0, 0) (it may lie before the image)
-      ao[i] = uint32_t(((b - b0) * cv.iH + ih0[i]) * cv.iW + iw0[i]) * uint32_t(cv.ldx);
+      // element offset of tap (0, 0) (it may lie before the base; modulo 2^32)
+      ao[i] = ((uint32_t(b - b0) * uint32_t(cv.iH) + uint32_t(ih0[i] - row0)) * uint32_t(cv.iW) + uint32_t(iw0[i])) *
+              uint32_t(cv.ldx);
     }
   } else {
     abase = long(m0) * lda;
@@ -130,7 +134,7 @@ gemm_f32_kernel(const float *__restrict__ A, const float *__restrict__ Bt, int M
     constexpr int d = decltype(setc)::value;
     const bool in = ks + c * 4 < K;  // K % 4 == 0: a chunk is inside or past the end
     if constexpr (CONV) {
-      const uint32_t toff = uint32_t(kh * cv.iW + kw) * uint32_t(cv.ldx) + ic;
+      const uint32_t toff = (uint32_t(kh) * uint32_t(cv.iW) + uint32_t(kw)) * uint32_t(cv.ldx) + ic;
 #pragma unroll
       for (int i = 0; i < ACH; ++i) {
         const bool ok = in && unsigned(ih0[i] + kh) < unsigned(cv.iH) && unsigned(iw0[i] + kw) < unsigned(cv.iW);
@@ -315,12 +319,12 @@ int auto_tile(int M, int N, int batch) {
 bool gemm_f32_ok(const void *A, const void *Bt, int K, long lda, long ldb, long sa, long sb, const ConvArgs *cv) {
   const bool b = K > 0 && K % 4 == 0 && ldb % 4 == 0 && sb % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)Bt % 16 == 0;
   // 32-bit byte offsets within a tile's 64 rows (a convolution's: within the
-  // images that 64 output pixels touch), below the out-of-range offset 2^31
+  // input rows that 64 output pixels touch), below the out-of-range offset 2^31
   const long rows = 64 * 4, lim = 0x7fffffffL;
   if (!b || long(ldb) * rows > lim || ldb < 0) return false;
   if (!cv) return lda % 4 == 0 && sa % 4 == 0 && lda >= 0 && lda * rows <= lim;
-  const long imgs = 64 / std::max(1, cv->oH * cv->oW) + 2;
-  return cv->iC % 4 == 0 && cv->ldx % 4 == 0 && imgs * cv->iH * cv->iW * cv->ldx * 4 <= lim;
+  const long span = conv_row_span(64, cv->B, cv->iH, cv->oH, cv->oW, cv->kH, cv->s, cv->p);
+  return cv->iC % 4 == 0 && cv->ldx % 4 == 0 && span * cv->iW * cv->ldx * 4 <= lim;
 }
 
 hipError_t gemm_f32(const float *A, const float *Bt, int M, int N, int K, long lda, long ldb, int batch, long sa,

@@ -34,6 +34,20 @@ inline int argmax_threads(long rows, int n) {
   return n >= 4096 || (n >= 2048 && rows <= std::max(256, n / 8)) ? 1024 : 256;
 }
 
+// Implicit-GEMM convolution: the input row, within its image, that the offsets
+// of a block of output pixels start from, for a first pixel in output row oh.
+__host__ __device__ __forceinline__ int conv_base_row(int oh, int iH, int s, int p) {
+  const int r = oh * s - p;
+  return r < 0 ? 0 : r < iH ? r : iH - 1;
+}
+// No fewer than the input rows, over all images, from there to the last one that
+// `pix` consecutive output pixels touch: they lie in (pix - 2) / oW + 2 output
+// rows, which start s input rows apart, or what an image leaves below its last.
+inline long conv_row_span(int pix, long B, long iH, long oH, long oW, long kH, long s, long p) {
+  const long step = std::max(s, iH - (oH - 1) * s);
+  return std::min(((pix - 2) / std::max(1L, oW) + 1) * step + kH + p, B * iH);
+}
+
 // Row-broadcast kernel: tpr threads per row, rpb rows per 256-thread
 // workgroup, gx x gy workgroups for rows of cpr 16-byte chunks; up to 32768
 // workgroups of one row in flight per thread, or 8192 of kRowsInFlight.

@@ -53,7 +53,32 @@ static void split(long rows, int threads) {
   if (next != rows) fail("rows", rows, threads, next);
 }
 
+// Every valid input row that any 64 consecutive output pixels touch lies within
+// the span from their base row.
+static void conv(int B, int iH, int iW, int k, int s, int p) {
+  const int oH = (iH + 2 * p - k) / s + 1, oW = (iW + 2 * p - k) / s + 1;
+  if (iH + 2 * p < k || iW + 2 * p < k) return;
+  const long M = long(B) * oH * oW, span = mh::conv_row_span(64, B, iH, oH, oW, k, s, p);
+  for (long m0 = 0; m0 < M; ++m0) {
+    const long b0 = m0 / (oH * oW), base = b0 * iH + mh::conv_base_row(int(m0 % (oH * oW) / oW), iH, s, p);
+    if (base < b0 * iH || base >= (b0 + 1) * iH) fail("base row", m0, base, iH);
+    for (long m = m0; m < m0 + 64 && m < M; ++m)
+      for (int kh = 0; kh < k; ++kh) {
+        const long ih = m % (oH * oW) / oW * s - p + kh, r = m / (oH * oW) * iH + ih;
+        if (ih >= 0 && ih < iH && (r < base || r >= base + span)) fail("row span", m0, r - base, span);
+      }
+  }
+}
+
 int main() {
+  for (int B : {1, 3})
+    for (int iH : {1, 2, 5, 8, 17})
+      for (int iW : {1, 3, 7, 31, 64, 100})
+        for (int k : {1, 2, 3, 5, 7})
+          for (int s : {1, 2, 3, 4})
+            for (int p : {0, 1, 2, 3, 6}) conv(B, iH, iW, k, s, p);
+  // an image of 1 GiB, 64 floats at 2048 x 2048, a few rows of which a tile sees
+  if (mh::conv_row_span(64, 4, 2048, 2048, 2048, 3, 1, 1) * 2048 * 64 * 4 > 1 << 24) fail("large image", 0, 0, 0);
   const long rows[] = {1, 2, 3, 5, 255, 1024, 1025, 65537, 99999, 8388609, 2139095040, 2139095041, 2147483000, 2147483646};
   for (long r : rows)
     for (int cpr : {1, 2, 3, 8, 100, 255, 256, 257, 5000, 3000000})

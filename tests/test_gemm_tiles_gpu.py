@@ -134,11 +134,12 @@ def test_f16_fixed_programs_bit_identical_to_general(tile, hip, monkeypatch):
         assert torch.equal(outs[0], outs[1]), f"tile {tile} act={act} resid={resid is not None} bias={use_bias}"
 
 
-@pytest.mark.parametrize("tile", [None, 300, 301, 302])
+@pytest.mark.parametrize("tile", [None, 300, 301, 302, 104])
 @pytest.mark.parametrize("M,K,N", [(65, 32, 64), (64, 36, 68), (31, 4, 33), (130, 100, 200), (1, 64, 5), (300, 516, 31)])
 @pytest.mark.parametrize("batched", [False, True])
 def test_f32_tiles(hip, monkeypatch, tile, M, K, N, batched):
-    """The fp32 kernel's tiles at their edges: one slab, an odd and an even
+    """The fp32 kernel's tiles, and the general kernel's chunked loader (104),
+    at their edges: one slab, an odd and an even
     number of 32-wide slabs, K tails of 4 values, ragged rows and columns, batch
     slices.  Against float64; a sum of K products rounds at most K times, each
     by 2^-24 of a partial sum, and M N outputs of standard normal operands stay
@@ -156,21 +157,50 @@ def test_f32_tiles(hip, monkeypatch, tile, M, K, N, batched):
 
 
 @pytest.mark.parametrize("B,iC,H,W,oC,k,s,p", [(2, 4, 9, 7, 33, 3, 1, 1), (1, 12, 8, 8, 64, 5, 2, 2), (3, 36, 5, 6, 20, 3, 2, 1),
-                                               (1, 64, 16, 16, 128, 3, 1, 1), (2, 32, 4, 4, 8, 1, 1, 0), (1, 8, 7, 7, 8, 7, 1, 3)])
-def test_f32_conv_columns(hip, B, iC, H, W, oC, k, s, p):
+                                               (1, 64, 16, 16, 128, 3, 1, 1), (2, 32, 4, 4, 8, 1, 1, 0), (1, 8, 7, 7, 8, 7, 1, 3),
+                                               (40, 8, 3, 2, 70, 3, 2, 1), (2, 16, 40, 37, 100, 3, 1, 1), (2, 4, 6, 1, 9, 1, 3, 2)])
+def test_f32_conv_columns(hip, B, iC, H, W, oC, k, s, p, monkeypatch):
     """The fp32 implicit-GEMM convolution's stepped (tap, channel) columns:
     channel counts below, at and above a 32-wide slab that divide it or not,
-    1x1 to 7x7 taps, strides, padding.  Against float64, bound as in
-    test_f32_tiles with K = k k iC."""
+    1x1 to 7x7 taps, strides, padding, tiles that cross image borders.  Against
+    float64, bound as in test_f32_tiles with K = k k iC, on every tile, which
+    all sum in one order: the same bits; and on the general kernel's chunked
+    loader."""
     import torch
     g = torch.Generator().manual_seed(iC * 10 + k)
     x, w, b = torch.randn(B, iC, H, W, generator=g), torch.randn(oC, iC, k, k, generator=g), torch.randn(oC, generator=g)
     ref = torch.nn.functional.conv2d(x.double(), w.double(), b.double(), stride=s, padding=p).permute(0, 2, 3, 1)
-    out = empty(tuple(ref.shape), synth.F32)
-    hip.conv2d_nhwc(x.permute(0, 2, 3, 1).contiguous().cuda(), w.permute(0, 2, 3, 1).contiguous().cuda(), b.cuda(), out, B,
-                    iC, H, W, oC, k, k, s, p)
     K = iC * k * k
-    assert float((out.cpu().double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24 + 1e-6
+    args = x.permute(0, 2, 3, 1).contiguous().cuda(), w.permute(0, 2, 3, 1).contiguous().cuda(), b.cuda()
+    outs = {}
+    for tile in (None, "300", "301", "302", "general"):
+        monkeypatch.delenv("MUNET_HIP_CONV_TILE", raising=False)
+        monkeypatch.delenv("MUNET_HIP_CONV_KERNEL", raising=False)
+        if tile:
+            monkeypatch.setenv("MUNET_HIP_CONV_KERNEL" if tile == "general" else "MUNET_HIP_CONV_TILE", tile)
+        out = empty(tuple(ref.shape), synth.F32)
+        hip.conv2d_nhwc(*args, out, B, iC, H, W, oC, k, k, s, p)
+        outs[tile] = out.cpu()
+        assert float((outs[tile].double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24 + 1e-6, tile
+    assert all(torch.equal(outs["300"], outs[t]) for t in (None, "301", "302"))
+
+
+def test_f32_conv_large_image(hip):
+    """An image of 1 GiB (its offsets are taken from the tile's first input
+    row): rows at both ends and in the middle against float64."""
+    import torch
+    C, H, W, oC = 64, 2048, 2048, 8
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(1, H, W, C, device="cuda", generator=g)
+    w, b = torch.randn(oC, 3, 3, C, device="cuda", generator=g), torch.randn(oC, device="cuda", generator=g)
+    out = empty((1, H, W, oC), synth.F32)
+    hip.conv2d_nhwc(x, w, b, out, 1, C, H, W, oC, 3, 3, 1, 1)
+    wd, K = w.cpu().double().permute(0, 3, 1, 2), 9 * C
+    for r in (0, 1, 1023, 1024, H - 2, H - 1):
+        lo, hi = max(r - 1, 0), min(r + 2, H)
+        xs = torch.nn.functional.pad(x[:, lo:hi].cpu().double().permute(0, 3, 1, 2), (1, 1, lo - (r - 1), r + 2 - hi))
+        ref = torch.nn.functional.conv2d(xs, wd, b.cpu().double())[0, :, 0].T
+        assert float((out[0, r].cpu().double() - ref).abs().max()) <= 6 * K ** 1.5 * 2.0 ** -24 + 1e-6, r
 
 
 @pytest.mark.parametrize("tile", list(range(220, 228)))
