@@ -104,6 +104,7 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // groups: move to the nearest tile whose wave-tile width is a multiple
   if (ep.stats_out && pipe_wave_cols(tile) % ep.stats_cols)
     tile = ep.stats_cols == 48 ? (dma ? 8 : 3) : ep.stats_cols == 64 ? (dma ? 9 : 0) : 2;
+  if (tile >= 20 && kind == PK_BIAS_NT) tile = 9;  // (forced: the many-stage tiles have no streamed program)
   if (tile >= 20) {
     // a forced tile that has not this program takes 64x64
     const bool ln = ep.ln_stats != nullptr, no = (ln && (tile == 23 || tile == 26)) || (!ep.stats_out && (tile == 21 || tile == 24));
