@@ -279,14 +279,14 @@ softmax_long_kernel(const typename Store<DT>::T *__restrict__ x, typename Store<
   const int tid = threadIdx.x;
   const typename Store<DT>::T *xr = x + long(blockIdx.x) * cols;
   float mx = -INFINITY;
-  for (int c = tid; c < cols; c += 1024) mx = fmaxf(mx, S::dec(xr[c]));
+  for (unsigned c = tid; c < unsigned(cols); c += 1024) mx = fmaxf(mx, S::dec(xr[c]));
   mx = wave_max(mx);
   if ((tid & 63) == 0) smx[tid >> 6] = mx;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < 16; ++w) mx = fmaxf(mx, smx[w]);
   double sum = 0.0;
-  for (int c = tid; c < cols; c += 1024) sum += exp(double(S::dec(xr[c])) - double(mx));
+  for (unsigned c = tid; c < unsigned(cols); c += 1024) sum += exp(double(S::dec(xr[c])) - double(mx));
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
   if ((tid & 63) == 0) ssum[tid >> 6] = sum;
@@ -295,7 +295,7 @@ softmax_long_kernel(const typename Store<DT>::T *__restrict__ x, typename Store<
 #pragma unroll
   for (int w = 0; w < 16; ++w) sum += ssum[w];
   typename Store<DT>::T *yr = y + long(blockIdx.x) * cols;
-  for (int c = tid; c < cols; c += 1024) yr[c] = S::enc(float(exp(double(S::dec(xr[c])) - double(mx)) / sum));
+  for (unsigned c = tid; c < unsigned(cols); c += 1024) yr[c] = S::enc(float(exp(double(S::dec(xr[c])) - double(mx)) / sum));
 }
 
 // Threads per row by its length: a wave to 512 values (eight per lane), 256
