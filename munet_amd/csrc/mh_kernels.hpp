@@ -113,7 +113,7 @@ hipError_t gemm_dma(int dt, const void *A, const void *Bt, int M, int N, int K, 
 // 7 128x128 3 stages, 8 128x96 4 stages, 9 128x128 2 stages, 10 128x96
 // 2 stages, 11 128x96 3 stages, 12 128x64 3 stages; eight waves 16 256x192
 // 2 stages, 17 128x96 4 stages, 19 128x288 3 stages; many stages 20 64x64, 21
-// 64x48, 22 64x96, 23 32x64, 24 32x48, 25 128x64, 26 32x32.
+// 64x48, 22 64x96, 23 32x64, 24 32x48, 25 128x64, 26 32x32, 27 128x128.
 bool gemm_pipe_ok(int dt, const void *A, const void *Bt, int M, int N, int K, long lda, long ldb, long sa, long sb);
 bool gemm_pipe_dma_ok(const void *A, const void *Bt, int M, int N, int K, long lda, long ldb);
 hipError_t gemm_pipe(int dt, const void *A, const void *Bt, int M, int N, int K, long lda, long ldb, int batch,

@@ -166,7 +166,8 @@ def test_attention_head_sizes(hip, dt, hd, B, H, T, causal, textbook):
     Tolerances, against rows of max |ctx| about 1: fp32 2e-5, the scores' sum
     error (hd 2^-24 |q||k| scale, about 1e-6) plus T sums; 16-bit: 2^-8 (bf16)
     and 2^-10 (fp16) of a score of magnitude 4 where the fp32 sum order moves a
-    rounding, and one rounding of p and of the result, 2e-2 in all."""
+    rounding, and one rounding of p and of the result: 2e-2 (bf16) and 4e-3
+    (fp16) in all."""
     import torch
     tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dt]
     N = B * H * T
@@ -191,7 +192,7 @@ def test_attention_head_sizes(hip, dt, hd, B, H, T, causal, textbook):
         s = s.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -float("inf"))
     ref = (torch.softmax(s, -1) @ vd).view(B, H, T, hd).permute(0, 2, 1, 3).reshape(B * T, H * hd)
     err = float((ctx.cpu().double() - ref).abs().max() / ref.abs().max())
-    assert err <= (2e-5 if dt == F32 else 2e-2), err
+    assert err <= {F32: 2e-5, F16: 4e-3, BF16: 2e-2}[dt], err
 
 
 def _textbook_oracle(q, k, v, B, H, T, hd, causal, textbook):
