@@ -25,18 +25,21 @@ int pipe_wave_cols(int tile) {
   }
 }
 
+TileEpi tile_epi(const EpiArgs &ep) { return ep.act == ACT_GELU ? TILE_GELU : ep.resid ? TILE_RESID : TILE_PLAIN; }
+
 // Automatic block tile (gemm_tiles.hpp).
 int block_tile(bool dma, int dt, const EpiArgs &ep, int M, int N, int K, int batch) {
-  return auto_tile(dma, dt == F16, ep.act == ACT_GELU ? TILE_GELU : ep.resid ? TILE_RESID : TILE_PLAIN, M, N, K, batch);
+  return auto_tile(dma, dt == F16, tile_epi(ep), M, N, K, batch);
 }
 
 // Small tiles with many stages (gemm_pipe_deep.hip) while they give at most
 // one workgroup per CU, the smallest first: below that count a smaller tile
 // spreads the same steps over more CUs (237 x 768 x 3072: 32x32 10.0 us, 32x64
 // 11.3, 64x64 13.0, 64x96 15.4), above it the workgroups take turns (512 x
-// 768 x 3072: 32x32 17.7, 32x64 11.5).  -1: none fits, the block tiles.
+// 768 x 3072: 32x32 17.7, 32x64 11.5).  Too short a K takes 64x64 (short_loop).
+// -1: none fits, the block tiles.
 // A tile's wave tiles must cover whole groups of the LayerNorm partials.
-int deep_tile(int kind, int M, int N, int batch, const EpiArgs &ep) {
+int deep_tile(int kind, int dt, int M, int N, int K, int batch, const EpiArgs &ep) {
   if (kind == PK_BIAS_NT || ep.mode == EPI_CONVT) return -1;
   const bool ln = ep.ln_stats != nullptr, st = ep.stats_out != nullptr;
   struct T { int tile, bm, bn; };
@@ -47,7 +50,7 @@ int deep_tile(int kind, int M, int N, int batch, const EpiArgs &ep) {
     if (t.bn == 48 && !st) continue;
     if (t.tile == 22 && N % 96) continue;
     if (st && pipe_wave_cols(t.tile) % ep.stats_cols) continue;
-    return t.tile;
+    return !ln && !st && short_loop(dt == F16, tile_epi(ep), M, N, K, batch) ? 2 : t.tile;
   }
   return -1;
 }
@@ -96,7 +99,7 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // 11.5 -> 10.4, up0 19.1 -> 15.1 against 128x64; the direct-to-LDS 128x128
   // 20-31 us)
   if (tile < 0 && ep.mode == EPI_CONVT) tile = 2;
-  if (tile < 0 && dma) tile = deep_tile(kind, M, N, batch, ep);
+  if (tile < 0 && dma) tile = deep_tile(kind, DT, M, N, K, batch, ep);
   if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = block_tile(dma, DT, ep, M, N, K, batch);
   if (tile >= 7 && !dma) tile = 0;
   if (tile == 19 && (M % 128 || N % 288)) tile = block_tile(dma, DT, ep, M, N, K, batch);

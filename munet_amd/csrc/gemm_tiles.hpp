@@ -58,6 +58,15 @@ inline double tile_time(const TileTime &t, int M, int N, int K, int batch, bool 
 //    and to K = 2048 at up to 192 tiles (64x64 | 27: 2048 x 2048 x 512 16.3 | 17.2,
 //    1000 x 2500 x 1024 17.8 | 19.5, 1536 x 2500 x 1024 21.7 | 21.0, 2000 x 2048 x
 //    2048 33.6 | 29.2);
+//    At K = 64, one step of the loop, 64x64 whatever the type (27 | 64x64:
+//    2048 x 2048 bias 7.1 | 6.3, 1100 x 2048 bias 6.6 | 5.2, fp16 residual at 256
+//    tiles 8.7 | 8.1);
+//  * more, with K <= 768 and N tiling evenly by 96 into at most two tiles per CU:
+//    register-staged 128x96, unless fp16's GELU (the sizes that the model below
+//    knows least: its loops are longer, and 128x288 filling half the chip had
+//    one shape.  The model's | 128x96, us: 8192 x 768 x 256 bias, fp16 12.2 |
+//    10.9, 4096 x 1152 x 512 bf16 GELU 14.1 | 12.5; bf16 GELU at K = 768 17.1 |
+//    17.5);
 //  * more: the least of kTileTimes (bf16 with a residual, 4096 x 5000 x 512:
 //    128x128 37.2, 256x192 50.3; fp16 GELU, 1100 x 5000 x 512: 128x64 22.3,
 //    two-stage 128x128 27.6);
@@ -75,8 +84,10 @@ inline int auto_tile(bool dma, bool f16, TileEpi epi, int M, int N, int K, int b
   const long t288 = long(M / 128) * (N / 288) * batch;
   if (dma && M % 128 == 0 && N % 288 == 0 && t288 >= 232 && t288 <= 256) return 19;
   if (dma && N % 96 == 0 && t96 <= 256) return 17;
+  if (dma && t128 > 128 && t128 <= 256 && K <= 64) return 2;
   if (dma && t128 > 128 && t128 <= 256)
     return f16 && epi == TILE_GELU && (K < 768 || (K < 2048 && t128 <= 192)) ? 2 : 27;
+  if (dma && t128 > 256 && K <= 768 && N % 96 == 0 && t96 <= 512 && !(f16 && epi == TILE_GELU)) return 3;
   if (dma && t128 > 256) {
     int best = 9;
     double best_t = 1e30;
@@ -93,6 +104,19 @@ inline int auto_tile(bool dma, bool f16, TileEpi epi, int M, int N, int K, int b
   if (N % 128 == 0 && t128 >= 640) return 0;
   if (N % 96 == 0) return 3;
   return (t128 >= 640 || (K >= 2048 && t128 >= 128)) ? 0 : (t64 >= 256 ? 1 : 2);
+}
+
+// Of a product that the many-stage tiles could take: whether its K is too short
+// for them to fill their stages, so that register-staged 64x64 is faster.  One
+// step (K = 64): yes (many-stage | 64x64, us, bf16 1 x 64 3.1 | 2.7, 2000 x 512
+// 4.2 | 3.5, 500 x 2048 4.2 | 3.5), but with fp16's roundings in the epilogue only
+// from about a tile per CU.  Two and three steps: from there too (K = 128 by up
+// to 7%, 192 by 4%), below it the smaller many-stage tiles use more CUs.  Rows of
+// N % 4 != 0 have no packed epilogue in 64x64 (6.3 against 4.0).
+inline bool short_loop(bool f16, TileEpi epi, int M, int N, int K, int batch) {
+  if (N % 4) return false;
+  const long t = long((M + 63) / 64) * ((N + 63) / 64) * batch;
+  return (K <= 64 && (!f16 || epi == TILE_PLAIN)) || (K <= 192 && t > 200);
 }
 
 }  // namespace mh

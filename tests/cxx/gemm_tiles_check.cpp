@@ -16,7 +16,10 @@ int main() {
       {true, TILE_GELU, 2048, 2048, 512, 2, 2},     {true, TILE_GELU, 1100, 5000, 512, 1, 2},
       {true, TILE_GELU, 8192, 4096, 512, 1, 1},     {true, TILE_GELU, 8192, 8192, 2048, 0, 9},
       {false, TILE_RESID, 4096, 5000, 512, 0, 9},   {false, TILE_RESID, 2000, 5000, 512, 1, 0},
-      {false, TILE_RESID, 8192, 2500, 1024, 0, 9},  {true, TILE_GELU, 8192, 2048, 8192, 9, 16}};
+      {false, TILE_RESID, 8192, 2500, 1024, 0, 9},  {true, TILE_GELU, 8192, 2048, 8192, 9, 16},
+      {false, TILE_PLAIN, 2048, 2048, 64, 2, 2},    {true, TILE_RESID, 2048, 2048, 64, 2, 2},
+      {true, TILE_PLAIN, 8192, 768, 256, 3, 3},     {false, TILE_PLAIN, 8192, 768, 128, 3, 3},
+      {true, TILE_GELU, 8192, 768, 256, 1, 2},      {false, TILE_GELU, 4096, 1152, 512, 3, 3}};
   for (const auto &w : want) {
     const int t = auto_tile(true, w.f16, w.epi, w.M, w.N, w.K, 1);
     if (t != w.a && t != w.b) {
@@ -24,6 +27,16 @@ int main() {
       return 1;
     }
   }
+  // where the many-stage tiles give way to 64x64
+  const struct { bool f16; TileEpi epi; int M, N, K; bool yes; } shorter[] = {
+      {false, TILE_PLAIN, 1, 64, 64, true},     {false, TILE_GELU, 500, 2048, 64, true}, {true, TILE_PLAIN, 33, 96, 64, true},
+      {true, TILE_GELU, 33, 96, 64, false},     {true, TILE_GELU, 500, 2048, 64, true},  {false, TILE_PLAIN, 2000, 512, 192, true},
+      {false, TILE_PLAIN, 2000, 512, 256, false}, {false, TILE_PLAIN, 1, 64, 128, false}, {false, TILE_PLAIN, 33, 97, 64, false}};
+  for (const auto &w : shorter)
+    if (short_loop(w.f16, w.epi, w.M, w.N, w.K, 1) != w.yes) {
+      std::printf("%d x %d x %d f16 %d epi %d: short loop %d\n", w.M, w.N, w.K, w.f16, w.epi, !w.yes);
+      return 1;
+    }
   for (int M : {1, 129, 4096, 100000})
     for (int N : {1, 288, 5000, 100000})
       for (int K : {64, 512, 8192, 1 << 20})
