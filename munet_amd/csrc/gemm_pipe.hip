@@ -25,11 +25,9 @@ int pipe_wave_cols(int tile) {
   }
 }
 
-TileEpi tile_epi(const EpiArgs &ep) { return ep.act == ACT_GELU ? TILE_GELU : ep.resid ? TILE_RESID : TILE_PLAIN; }
-
-// Automatic block tile (gemm_tiles.hpp).
-int block_tile(bool dma, int dt, const EpiArgs &ep, int M, int N, int K, int batch) {
-  return auto_tile(dma, dt == F16, tile_epi(ep), M, N, K, batch);
+TileEpi tile_epi(int dt, int kind, bool packed, const EpiArgs &ep) {
+  if (packed && kind == PK_GENERAL && !(dt == F16 && ep.act == ACT_GELU)) return TILE_GENERAL;
+  return ep.act == ACT_GELU ? TILE_GELU : ep.resid ? TILE_RESID : TILE_PLAIN;
 }
 
 // Small tiles with many stages (gemm_pipe_deep.hip) while they give at most
@@ -39,7 +37,7 @@ int block_tile(bool dma, int dt, const EpiArgs &ep, int M, int N, int K, int bat
 // 768 x 3072: 32x32 17.7, 32x64 11.5).  Too short a K takes 64x64 (short_loop).
 // -1: none fits, the block tiles.
 // A tile's wave tiles must cover whole groups of the LayerNorm partials.
-int deep_tile(int kind, int dt, int M, int N, int K, int batch, const EpiArgs &ep) {
+int deep_tile(int kind, bool packed, bool f16, TileEpi epi, int M, int N, int K, int batch, const EpiArgs &ep) {
   if (kind == PK_BIAS_NT || ep.mode == EPI_CONVT) return -1;
   const bool ln = ep.ln_stats != nullptr, st = ep.stats_out != nullptr;
   struct T { int tile, bm, bn; };
@@ -50,7 +48,7 @@ int deep_tile(int kind, int dt, int M, int N, int K, int batch, const EpiArgs &e
     if (t.bn == 48 && !st) continue;
     if (t.tile == 22 && N % 96) continue;
     if (st && pipe_wave_cols(t.tile) % ep.stats_cols) continue;
-    return !ln && !st && short_loop(dt == F16, tile_epi(ep), M, N, K, batch) ? 2 : t.tile;
+    return !ln && !st && short_loop(packed, f16, epi, M, N, K, batch) ? 2 : t.tile;
   }
   return -1;
 }
@@ -60,18 +58,22 @@ bool fixed_tile(int tile) {
   return (tile >= 0 && tile <= 3) || tile == 8 || tile == 9 || tile == 16 || tile == 17 || tile == 19 || tile >= 20;
 }
 
+// Whether the epilogue stores an output row four values at a time.
+bool packed_rows(int dt, int N, int batch, long sc, const EpiArgs &ep) {
+  if ((dt != BF16 && dt != F16) || N % 4 || ep.mode == EPI_CONVT || (ep.resid && (ep.ldr & 3))) return false;
+  if (ep.mode == EPI_HEADSPLIT)
+    return (ep.hd & 3) == 0 && ((uintptr_t)ep.outs[0] & 7) == 0 && ((uintptr_t)ep.outs[1] & 7) == 0 &&
+           ((uintptr_t)ep.outs[2] & 7) == 0;
+  return ((uintptr_t)ep.out & 7) == 0 && (ep.ldc & 3) == 0 && (batch == 1 || (sc & 3) == 0);
+}
+
 // The epilogue program for these arguments: a fixed program for the
 // combinations the engine emits (bf16, 8-byte aligned destination, bias
 // after the matmul rounding), else PK_GENERAL; -1 for a folded LayerNorm
 // outside the fixed programs (it has no general form).
 int pipe_kind(int dt, int N, int batch, long sc, const EpiArgs &ep) {
   const bool fold = ep.ln_stats || ep.stats_out;
-  const bool fast = (dt == BF16 || dt == F16) && N % 4 == 0 && ep.mode != EPI_CONVT && (!ep.resid || (ep.ldr & 3) == 0);
-  const bool al8 = ep.mode == EPI_HEADSPLIT
-                       ? (ep.hd & 3) == 0 && ((uintptr_t)ep.outs[0] & 7) == 0 && ((uintptr_t)ep.outs[1] & 7) == 0 &&
-                             ((uintptr_t)ep.outs[2] & 7) == 0
-                       : ((uintptr_t)ep.out & 7) == 0 && (ep.ldc & 3) == 0 && (batch == 1 || (sc & 3) == 0);
-  if (!fast || !al8 || (ep.bias && ep.bias_first)) return fold ? -1 : PK_GENERAL;
+  if (!packed_rows(dt, N, batch, sc, ep) || (ep.bias && ep.bias_first)) return fold ? -1 : PK_GENERAL;
   const bool hb = ep.bias != nullptr, hr = ep.resid != nullptr;
   if (fold && dt != BF16) return -1;  // the folded LayerNorm programs are bf16 only
   if (ep.ln_stats) {
@@ -86,7 +88,8 @@ int pipe_kind(int dt, int N, int batch, long sc, const EpiArgs &ep) {
 template <int DT>
 hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long lda, long ldb, int batch, long sa,
                      long sb, long sc, const EpiArgs &ep, int tile, int kind, hipStream_t st) {
-  const bool dma = gemm_pipe_dma_ok(A, Bt, M, N, K, lda, ldb);
+  const bool dma = gemm_pipe_dma_ok(A, Bt, M, N, K, lda, ldb), packed = packed_rows(DT, N, batch, sc, ep);
+  const TileEpi epi = tile_epi(DT, kind, packed, ep);
   // a folded LayerNorm exists only in the fixed programs: a forced tile
   // without the program takes the automatic choice
   // a large streamed output (the vocabulary head): direct-to-LDS 128x128,
@@ -99,10 +102,10 @@ hipError_t launch_dt(const void *A, const void *Bt, int M, int N, int K, long ld
   // 11.5 -> 10.4, up0 19.1 -> 15.1 against 128x64; the direct-to-LDS 128x128
   // 20-31 us)
   if (tile < 0 && ep.mode == EPI_CONVT) tile = 2;
-  if (tile < 0 && dma) tile = deep_tile(kind, DT, M, N, K, batch, ep);
-  if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = block_tile(dma, DT, ep, M, N, K, batch);
+  if (tile < 0 && dma) tile = deep_tile(kind, packed, DT == F16, epi, M, N, K, batch, ep);
+  if (tile < 0 || (kind >= PK_LN_BIAS && !fixed_tile(tile))) tile = auto_tile(dma, packed, DT == F16, epi, M, N, K, batch);
   if (tile >= 7 && !dma) tile = 0;
-  if (tile == 19 && (M % 128 || N % 288)) tile = block_tile(dma, DT, ep, M, N, K, batch);
+  if (tile == 19 && (M % 128 || N % 288)) tile = auto_tile(dma, packed, DT == F16, epi, M, N, K, batch);
   // LayerNorm partials of stats_cols columns need wave tiles that cover whole
   // groups: move to the nearest tile whose wave-tile width is a multiple
   if (ep.stats_out && pipe_wave_cols(tile) % ep.stats_cols)

@@ -5,7 +5,9 @@
 
 namespace mh {
 
-enum TileEpi { TILE_PLAIN, TILE_GELU, TILE_RESID };  // no more than a bias; an activation with exponentials; a residual
+// Epilogue: no more than a bias; an activation with exponentials; a residual;
+// packed rows in the general program (a ReLU, an activation without a bias).
+enum TileEpi { TILE_PLAIN, TILE_GELU, TILE_RESID, TILE_GENERAL };
 
 // A tile's time over n = its tiles in the product: rounds(n) (k K + epi[type]) +
 // launch, in us, where a round is per_cu tiles on each of 256 CUs and a last
@@ -13,10 +15,14 @@ enum TileEpi { TILE_PLAIN, TILE_GELU, TILE_RESID };  // no more than a bias; an 
 // `over` to 1 (per_cu = 1: `half` to 1).  Fitted to 16 (N, K) of 512 to 8192 by
 // 9 M of 500 to 8192, three epilogues and both types (weights and rows in L2
 // or not as they fit): 2 to 4% rms per tile, and the tile of least predicted time
-// takes 0.4% longer than the fastest on average, 9% at worst.
+// takes 0.4% longer than the fastest on average, 9% at worst.  The general program
+// counts as a residual in bf16 and as a GELU in fp16, whose roundings it makes
+// value by value (ReLU, 10 products of K 64 to 2048: 1.4% and 2.1% over the
+// fastest on average; as no more than a bias fp16 11%, 1100 x 8192 x 512 37.9 us
+// on 256x192 against 24.6 on 128x64).
 struct TileTime {
   int tile, bm, bn, per_cu;
-  double half, over, k, epi[3][2], launch;  // epi[TileEpi][fp16]
+  double half, over, k, epi[3][2], launch;  // epi[TileEpi below TILE_GENERAL][fp16]
 };
 constexpr TileTime kTileTimes[6] = {
     {0, 128, 128, 2, 0.50, 0.80, 0.0143, {{3.6, 4.9}, {4.7, 19.8}, {6.3, 9.1}}, 5.5},
@@ -32,11 +38,31 @@ inline double tile_time(const TileTime &t, int M, int N, int K, int batch, bool 
   double rounds = double(n / round);
   if (rem && t.per_cu == 1) rounds += t.half + (1 - t.half) * double(rem) / 256;
   else if (rem) rounds += rem <= 256 ? t.half : t.over + (1 - t.over) * double(rem - 256) / 256;
-  return rounds * (t.k * K + t.epi[epi][f16]) + t.launch;
+  const TileEpi cost = epi != TILE_GENERAL ? epi : f16 ? TILE_GELU : TILE_RESID;
+  return rounds * (t.k * K + t.epi[cost][f16]) + t.launch;
 }
 
-// dma: the operands allow direct-to-LDS loads (K % 64 == 0).  Tile codes as in
-// gemm_pipe.hpp.
+// Output rows that cannot be stored four at a time (N % 4 != 0, a destination or
+// residual off 8 bytes): the epilogue goes value by value and takes longer than
+// most loops, so that tiles whose workgroups overlap it, several to a CU, win
+// over the wide ones until the loop is long.  Register-staged 64x64 for short
+// loops (always at K <= 128, fp16 longer, as its roundings are), 128x64 between,
+// 128x128 for the long ones; at up to 256 128x128 tiles the many-stage 128x128
+// for the long ones.  Us, 64x64 | 128x64 | 128x128 | two-stage 128x128 | 256x192:
+// bf16 GELU, 1100 x 8193 x 256 22.3 | 22.2 | 30.4 | 28.4 | 51.4; fp16 bias, 2000 x
+// 5001 x 512 33.5 | 35.0 | 48.2 | 48.0 | 67.8, 1100 x 8193 x 128 20.4 | 22.7 | 35.2 |
+// 33.2 | 59.8; bf16 bias, 4096 x 4098 x 2048 114 | 101 | 94 | 99 | 113; 1500 x 2049 x
+// 2048 30.2 | 27.1 | 27.1, many-stage 22.8.
+inline int unpacked_tile(bool f16, TileEpi epi, int K, long t128) {
+  const bool slow = epi == TILE_RESID || (f16 && epi == TILE_GELU);
+  if (t128 <= 256) return K < (f16 ? 2049 : 1024) ? 2 : 27;
+  if (t128 >= 512 && K >= (slow ? 4096 : 2048)) return 0;
+  return K <= 128 || (f16 && K < 2048 && (slow || K <= 512)) ? 2 : 1;
+}
+
+// dma: the operands allow direct-to-LDS loads (K % 64 == 0).  packed: output rows
+// are stored four values at a time (more than 128 128x128 tiles that are not:
+// unpacked_tile).  Tile codes as in gemm_pipe.hpp.
 //  * M tiling evenly by 256 and N by 192 into 232..256 tiles (the decoder's FFN
 //    up, 4096 x 3072: 256): direct-to-LDS 256x192 with eight waves, one
 //    workgroup per CU (FFN up in the forward 33.1 -> 31.1 us; QKV, 192 tiles,
@@ -62,7 +88,7 @@ inline double tile_time(const TileTime &t, int M, int N, int K, int batch, bool 
 //    2048 x 2048 bias 7.1 | 6.3, 1100 x 2048 bias 6.6 | 5.2, fp16 residual at 256
 //    tiles 8.7 | 8.1);
 //  * more, with K <= 768 and N tiling evenly by 96 into at most two tiles per CU:
-//    register-staged 128x96, unless fp16's GELU (the sizes that the model below
+//    register-staged 128x96, unless fp16's GELU or general program (the sizes that the model below
 //    knows least: its loops are longer, and 128x288 filling half the chip had
 //    one shape.  The model's | 128x96, us: 8192 x 768 x 256 bias, fp16 12.2 |
 //    10.9, 4096 x 1152 x 512 bf16 GELU 14.1 | 12.5; bf16 GELU at K = 768 17.1 |
@@ -75,10 +101,11 @@ inline double tile_time(const TileTime &t, int M, int N, int K, int batch, bool 
 //    128x64 / 64x64 by tile count.
 // (The vocabulary head, a non-temporal output, takes direct-to-LDS 128x128
 // with two stages.)
-inline int auto_tile(bool dma, bool f16, TileEpi epi, int M, int N, int K, int batch) {
+inline int auto_tile(bool dma, bool packed, bool f16, TileEpi epi, int M, int N, int K, int batch) {
   const long t128 = long((M + 127) / 128) * ((N + 127) / 128) * batch;
   const long t96 = long((M + 127) / 128) * ((N + 95) / 96) * batch;
   const long t64 = long((M + 127) / 128) * ((N + 63) / 64) * batch;
+  if (dma && !packed && t128 > 128) return unpacked_tile(f16, epi, K, t128);
   const long t192w = long(M / 256) * (N / 192) * batch;
   if (dma && M % 256 == 0 && N % 192 == 0 && t192w >= 232 && t192w <= 256) return 16;
   const long t288 = long(M / 128) * (N / 288) * batch;
@@ -87,7 +114,7 @@ inline int auto_tile(bool dma, bool f16, TileEpi epi, int M, int N, int K, int b
   if (dma && t128 > 128 && t128 <= 256 && K <= 64) return 2;
   if (dma && t128 > 128 && t128 <= 256)
     return f16 && epi == TILE_GELU && (K < 768 || (K < 2048 && t128 <= 192)) ? 2 : 27;
-  if (dma && t128 > 256 && K <= 768 && N % 96 == 0 && t96 <= 512 && !(f16 && epi == TILE_GELU)) return 3;
+  if (dma && t128 > 256 && K <= 768 && N % 96 == 0 && t96 <= 512 && !(f16 && (epi == TILE_GELU || epi == TILE_GENERAL))) return 3;
   if (dma && t128 > 256) {
     int best = 9;
     double best_t = 1e30;
@@ -111,11 +138,13 @@ inline int auto_tile(bool dma, bool f16, TileEpi epi, int M, int N, int K, int b
 // step (K = 64): yes (many-stage | 64x64, us, bf16 1 x 64 3.1 | 2.7, 2000 x 512
 // 4.2 | 3.5, 500 x 2048 4.2 | 3.5), but with fp16's roundings in the epilogue only
 // from about a tile per CU.  Two and three steps: from there too (K = 128 by up
-// to 7%, 192 by 4%), below it the smaller many-stage tiles use more CUs.  Rows of
-// N % 4 != 0 have no packed epilogue in 64x64 (6.3 against 4.0).
-inline bool short_loop(bool f16, TileEpi epi, int M, int N, int K, int batch) {
-  if (N % 4) return false;
+// to 7%, 192 by 4%), below it the smaller many-stage tiles use more CUs.  Rows
+// that are not packed: only instead of the largest, 128x64, and to a longer K,
+// as 64x64 overlaps their epilogues (500 x 2049 x 64, fp16 bias 16% faster, bf16
+// 11%; even at K = 512 in bf16 and 1024 in fp16).
+inline bool short_loop(bool packed, bool f16, TileEpi epi, int M, int N, int K, int batch) {
   const long t = long((M + 63) / 64) * ((N + 63) / 64) * batch;
+  if (!packed) return t > 256 && K < (f16 ? 1024 : 512);
   return (K <= 64 && (!f16 || epi == TILE_PLAIN)) || (K <= 192 && t > 200);
 }
 
