@@ -139,12 +139,13 @@ inline int auto_tile(bool dma, bool packed, bool f16, TileEpi epi, int M, int N,
 // 4.2 | 3.5, 500 x 2048 4.2 | 3.5), but with fp16's roundings in the epilogue only
 // from about a tile per CU.  Two and three steps: from there too (K = 128 by up
 // to 7%, 192 by 4%), below it the smaller many-stage tiles use more CUs.  Rows
-// that are not packed: only instead of the largest, 128x64, and to a longer K,
+// that are not packed: from about a tile per CU at K = 64 (16 x 250 x 250, bf16 6.5 |
+// 5.9), and instead of the largest many-stage tile, 128x64, to a longer K,
 // as 64x64 overlaps their epilogues (500 x 2049 x 64, fp16 bias 16% faster, bf16
 // 11%; even at K = 512 in bf16 and 1024 in fp16).
 inline bool short_loop(bool packed, bool f16, TileEpi epi, int M, int N, int K, int batch) {
   const long t = long((M + 63) / 64) * ((N + 63) / 64) * batch;
-  if (!packed) return t > 256 && K < (f16 ? 1024 : 512);
+  if (!packed) return t > 256 ? K < (f16 ? 1024 : 512) : t > 200 && K <= 64;
   return (K <= 64 && (!f16 || epi == TILE_PLAIN)) || (K <= 192 && t > 200);
 }
 

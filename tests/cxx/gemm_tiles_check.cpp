@@ -46,7 +46,8 @@ int main() {
       {false, TILE_PLAIN, 1, 64, 64, true},     {false, TILE_GELU, 500, 2048, 64, true}, {true, TILE_PLAIN, 33, 96, 64, true},
       {true, TILE_GELU, 33, 96, 64, false},     {true, TILE_GELU, 500, 2048, 64, true},  {false, TILE_PLAIN, 2000, 512, 192, true},
       {false, TILE_PLAIN, 2000, 512, 256, false}, {false, TILE_PLAIN, 1, 64, 128, false}, {false, TILE_PLAIN, 33, 97, 64, false},
-      {true, TILE_PLAIN, 500, 2049, 512, true}, {true, TILE_PLAIN, 500, 2049, 1024, false}};
+      {true, TILE_PLAIN, 500, 2049, 512, true}, {true, TILE_PLAIN, 500, 2049, 1024, false},
+      {false, TILE_PLAIN, 4000, 250, 64, true}, {false, TILE_PLAIN, 4000, 250, 128, false}};
   for (const auto &w : shorter)
     if (short_loop(w.N % 4 == 0, w.f16, w.epi, w.M, w.N, w.K, 1) != w.yes) {
       std::printf("%d x %d x %d f16 %d epi %d: short loop %d\n", w.M, w.N, w.K, w.f16, w.epi, !w.yes);

@@ -215,7 +215,7 @@ def test_deep_tiles(tile, hip, orc, monkeypatch):
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (33, 96, 128), (256, 1024, 64), (257, 1024, 64), (500, 2048, 192), (512, 768, 256),
                                    (2048, 768, 64), (2049, 768, 64), (300, 4096, 64), (1900, 2056, 128), (4096, 1024, 192), (1500, 2048, 768), (600, 4096, 2048),
                                    (1100, 5000, 64), (1536, 4096, 128), (2048, 3072, 192), (2100, 4040, 320),
-                                   (2000, 516, 64), (500, 2044, 192), (33, 97, 64), (500, 2049, 192), (1100, 2501, 256), (1000, 2501, 1024), (2000, 2050, 64), (1100, 8193, 512), (1100, 8195, 2048), (1100, 2048, 64), (8192, 768, 256), (8100, 864, 448)])
+                                   (2000, 516, 64), (500, 2044, 192), (33, 97, 64), (500, 2049, 192), (4000, 250, 64), (1100, 2501, 256), (1000, 2501, 1024), (2000, 2050, 64), (1100, 8193, 512), (1100, 8195, 2048), (1100, 2048, 64), (8192, 768, 256), (8100, 864, 448)])
 def test_deep_tile_choice_bits(M, N, K, hip, monkeypatch):
     """Both sides of each border of the small-tile choice (at most one tile per
     CU) give the 128x128 kernel's bits, bias + GELU, bias + residual and ReLU."""
